@@ -1,0 +1,103 @@
+"""GPU tests of the MFMA GEMMs by row count: the weight-streaming kernel of few
+rows, at the edges of its 16-row tiles and of its column tiles, and with K
+that is not a whole 128-byte unit or leaves some of a workgroup's waves
+without one.
+
+Against float64 on the same inputs: an f32 sum of K products in any order is
+within K 2^-24 sum |a| |b| of the exact one.  A 16-bit output adds half an ulp:
+BF16 has 8 significant bits and F16 has 11, so that is at most 2^-8 and 2^-11 of
+the value (just above a power of two), and 2^-25 below F16's normal range.  The fused
+epilogues and the int8 GEMM are held bit for bit.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from vibe_compiler_amd import backend
+
+    ctx = backend.Context(0)
+    yield ctx
+    ctx.close()
+
+
+@pytest.fixture(scope="module")
+def B():
+    from vibe_compiler_amd import backend
+
+    return backend
+
+
+def _check(got, a, b, half_ulp):
+    """got [m, n] against a [m, k] . b [n, k]^T in float64, element by element."""
+    a, b = a.double(), b.double()
+    ref, mag = a @ b.t(), a.abs() @ b.abs().t()
+    bound = a.shape[1] * 2.0 ** -24 * mag
+    bound = bound + half_ulp * (ref.abs() + bound) + (2.0 ** -25 if half_ulp else 0.0)
+    over = (got.double() - ref).abs() - bound
+    assert float(over.max()) <= 0, float(over.max())
+
+
+ROWS = [(1, 128, 4096, 3), (15, 130, 96, 2), (16, 16, 32, 3), (17, 4096, 160, 3), (31, 33, 8192, 2), (32, 8192, 96, 3),
+        (33, 1000, 544, 2), (48, 10272, 64, 3), (63, 20, 2080, 3), (64, 12288, 128, 2), (64, 640, 1024, 3)]
+
+
+@pytest.mark.parametrize("m,n,k,fmt", ROWS)
+def test_gemm_rows_vs_float64(hip, B, m, n, k, fmt):
+    print("[gemm rows]", m, n, k, fmt, flush=True)
+    dt, half_ulp = (torch.bfloat16, 2.0 ** -8) if fmt == B.BF16 else (torch.float16, 2.0 ** -11)
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n * 3 + k)
+    a = torch.randn(m, k, generator=g, device="cuda").to(dt)
+    b = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(dt)
+    out = torch.full((m * n + 512,), 7.5, device="cuda")
+    hip.gemm_mfma(a, b, out, m, k, n, in_fmt=fmt, out_fmt=B.F32, rhs_t=True)
+    _check(out[:m * n].view(m, n), a, b, 0.0)
+    assert torch.all(out[m * n:] == 7.5)
+    # an output that no vector store is aligned for
+    for shift in (0, 1):
+        outn = torch.full((m * n + 512,), 7.5, dtype=dt, device="cuda")
+        view = outn[shift:shift + m * n]
+        hip.gemm_mfma(a, b, view, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
+        _check(view.view(m, n), a, b, half_ulp)
+        assert torch.all(outn[:shift] == 7.5) and torch.all(outn[shift + m * n:] == 7.5)
+    # the narrowed product plus a residual, in place, is the Add command's sum
+    r = torch.randn(m, n, generator=g, device="cuda").to(dt)
+    ref = torch.empty_like(r)
+    hip.elementwise("Add", fmt, view.clone().view(m, n), ref, r)
+    hip.gemm_mfma_residual(a, b, r, r, m, k, n, in_fmt=fmt, rhs_t=True)
+    assert torch.equal(r.view(torch.int16), ref.view(torch.int16))
+    if n % 16 == 0:  # SwiGLU of n features
+        wu = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(dt)
+        gate, up, ref, got = (torch.empty(m, n, dtype=dt, device="cuda") for _ in range(4))
+        hip.gemm_mfma(a, b, gate, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
+        hip.gemm_mfma(a, wu, up, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
+        hip.silu_mul(gate, up, ref, fmt=fmt)
+        packed = torch.empty(2 * n, k, dtype=dt, device="cuda")
+        hip.interleave_gate_up(b, wu, packed)
+        hip.gemm_mfma_swiglu(a, packed, got, m, k, n, in_fmt=fmt)
+        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 100, 64), (16, 4096, 1024), (33, 1001, 4160), (64, 12288, 192)])
+@pytest.mark.parametrize("rt", [False, True])
+def test_gemm_i8_rows_bit_exact(hip, B, m, n, k, rt):
+    print("[gemm i8 rows]", m, n, k, rt, flush=True)
+    rng = np.random.default_rng(m + n + k)
+    a = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    b = rng.integers(-127, 128, (n, k)).astype(np.int8)
+    scale = rng.uniform(0.001, 0.01, n).astype(np.float32)
+    acc_ref = a.astype(np.int64) @ b.astype(np.int64).T
+    y = torch.zeros(m * n + 64, dtype=torch.bfloat16, device="cuda")
+    acc = torch.zeros(m * n + 64, dtype=torch.int32, device="cuda")
+    rhs = b if rt else np.ascontiguousarray(b.T)
+    hip.gemm_i8(torch.from_numpy(a).cuda(), torch.from_numpy(rhs).cuda(), torch.from_numpy(scale).cuda(), y, m, k, n,
+                acc_out=acc, rhs_t=rt)
+    assert np.array_equal(acc[:m * n].view(m, n).cpu().numpy(), acc_ref)
+    yref = torch.from_numpy(acc_ref.astype(np.float32) * scale).to(torch.bfloat16)
+    assert torch.equal(y[:m * n].view(m, n).cpu(), yref)
+    assert torch.all(acc[m * n:] == 0) and torch.all(y[m * n:] == 0)

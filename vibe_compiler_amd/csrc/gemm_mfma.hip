@@ -26,7 +26,8 @@
 // (SwiGLU) and 128x192 tiles run on a 4-wave kernel instead (one wave per
 // SIMD, K slices moved by LDS DMA into a ring of 128 KiB), and long-K grids
 // of at most one round of 128x128 tiles split K over 4 workgroups of
-// 256x256 tiles with a fold launch.
+// 256x256 tiles with a fold launch.  Products of few rows go to the
+// weight-streaming kernel of gemm_skinny.hip.
 //
 // int8 semantics (no reference implementation exists; the closed form on the
 // reference's conversion routes): acc = sum_k int32(a)*int32(b) exactly
@@ -34,14 +35,13 @@
 // f32_RNE(acc) * scale[n])) -- int32_fp32 route, CT Mul, fp32_bf16 route
 // (lib/Wafer/Target/TargetFormat.cpp:174,192).  Integer sums are
 // order-independent, so the result is bit-exact.
-#include "common.h"
+#include "gemm_common.h"
 
 #include <type_traits>
 
 namespace wafer {
 namespace {
 
-enum { KIND_BF16 = 0, KIND_F16 = 1, KIND_I8 = 2 };
 typedef int v2i32 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) v2i32 lds_v2i32;
 constexpr int BKB = 64;  // K bytes must be a multiple of the smaller LDS stage
@@ -69,33 +69,6 @@ __device__ inline i32x16 mfma<KIND_I8>(u32x4 a, u32x4 b, i32x16 c) {
                                                __builtin_bit_cast(i32x4, b), c, 0, 0, 0);
 }
 
-// Epilogue selectors.
-// OUT_SWIGLU (bf16 or f16): the rhs rows come in 32-row groups, 16 gate rows
-// then the 16 up rows of the same features, and y[m, f] =
-// T(silu_mul(T(gate), T(up))) over N/2 features, T the storage format (the narrowed
-// products, then the silu_mul region).  In a 32x32 MFMA tile the gate
-// values of 16 features sit in lanes l32 < 16 and their up values in lanes
-// l32 + 16; one v_permlane16_swap per register pair brings both to one
-// lane (swiglu_pair).
-// OUT_NARROW_RES: the narrowed product plus a residual tensor of the same
-// format and shape, y = Add(narrow(acc), res) -- the GEMM's narrow output
-// followed by the CT Add command, bit for bit (y may be res itself: every
-// element is read before it is written, by the same lane).
-enum { OUT_F32 = 0, OUT_NARROW = 1, OUT_I8_DEQUANT = 2, OUT_SWIGLU = 3, OUT_NARROW_RES = 4 };
-
-// f16 -> f32 by v_cvt_f32_f16: exact for every finite f16 (subnormals
-// included, f16 denormals are on); a NaN keeps a NaN, and the sum it enters
-// narrows to the canonical f16 NaN either way, so the residual sum matches
-// the portable widening bit for bit.
-__device__ inline float widen_f16(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
-// f32 -> f16 by v_cvt_f16_f32 in the default round-to-nearest-even mode, with
-// gradual underflow and overflow to +-inf; a NaN narrows to the canonical
-// 0x7e00 as f32_to_f16 does.
-__device__ inline uint16_t narrow_f16(float x) {
-  x = f32_rounded(x);
-  return x != x ? (uint16_t)0x7e00u : __builtin_bit_cast(uint16_t, (_Float16)x);
-}
-
 // SwiGLU from accumulator registers r and r + 1 (r even: rows q and q + 1)
 // of a 32x32 tile whose columns 0..15 are gate and 16..31 up features:
 // v_permlane16_swap exchanges lanes 16..31 of `a` with lanes 0..15 of `b`
@@ -116,22 +89,6 @@ __device__ inline uint16_t swiglu_pair(float a, float b) {
     return (uint16_t)bf16x2_rne(y, y);
   }
 }
-
-struct GemmArgs {
-  const uint8_t *a;    // [M, K] elements, K-contiguous
-  const uint8_t *bt;   // [N, K] ([K, N] for the BKN int8 kernel)
-  void *y;             // [M, N]
-  int32_t *acc_out;    // int8 only, optional [M, N]
-  const float *scale;  // int8 only, [N]
-  int m, n, kbytes;    // K in bytes
-  int tiles_m, tiles_n;  // ceil(M / BM), ceil(N / BN)
-  const uint16_t *res;   // OUT_NARROW_RES only, [M, N]
-  // split-K (4-wave kernel only): ksplit > 1 workgroups per tile each take
-  // kbytes / ksplit of K and store f32 partial tiles to part [ksplit, M, N],
-  // which a fold launch adds in split order
-  int ksplit;
-  float *part;
-};
 
 // XCD-aware tile order: workgroup ids are dealt round-robin over the 8
 // XCDs; the ids one XCD receives cover a 4 x 8 block of output tiles when the
@@ -1344,7 +1301,10 @@ int prepare_split(wafer_hip_context *ctx, GemmArgs &args) {
 }
 
 template <int KIND, int OUT>
-int launch_gemm(hipStream_t st, GemmArgs args) {
+int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
+  const hipStream_t st = ctx->stream;
+  if (gemm_is_skinny(args.m))
+    return launch_gemm_skinny<KIND, OUT>(st, args, ctx->cu_count > 0 ? ctx->cu_count : 256);
   // 128-byte K stages where K allows (half the stage barriers per FLOP)
   return args.kbytes % 128 == 0 ? launch_gemm_sb<KIND, OUT, 128>(st, args) : launch_gemm_sb<KIND, OUT, 64>(st, args);
 }
@@ -1418,10 +1378,10 @@ extern "C" int wafer_hip_gemm_mfma(wafer_hip_context *ctx, const void *lhs, cons
   WAFER_TRY(prepare_split(ctx, args));
   const bool f32 = out_format == WAFER_FMT_F32;
   if (in_format == WAFER_FMT_BF16)
-    return f32 ? launch_gemm<KIND_BF16, OUT_F32>(ctx->stream, args)
-               : launch_gemm<KIND_BF16, OUT_NARROW>(ctx->stream, args);
-  return f32 ? launch_gemm<KIND_F16, OUT_F32>(ctx->stream, args)
-             : launch_gemm<KIND_F16, OUT_NARROW>(ctx->stream, args);
+    return f32 ? launch_gemm<KIND_BF16, OUT_F32>(ctx, args)
+               : launch_gemm<KIND_BF16, OUT_NARROW>(ctx, args);
+  return f32 ? launch_gemm<KIND_F16, OUT_F32>(ctx, args)
+             : launch_gemm<KIND_F16, OUT_NARROW>(ctx, args);
 }
 
 extern "C" int wafer_hip_gemm_mfma_residual(wafer_hip_context *ctx, const void *lhs, const void *rhs,
@@ -1439,8 +1399,8 @@ extern "C" int wafer_hip_gemm_mfma_residual(wafer_hip_context *ctx, const void *
   GemmArgs args{(const uint8_t *)lhs, bt, dst, nullptr, nullptr, (int)m, (int)n, (int)(k * 2), 0, 0,
                 (const uint16_t *)residual};
   WAFER_TRY(prepare_split(ctx, args));
-  return in_format == WAFER_FMT_BF16 ? launch_gemm<KIND_BF16, OUT_NARROW_RES>(ctx->stream, args)
-                                     : launch_gemm<KIND_F16, OUT_NARROW_RES>(ctx->stream, args);
+  return in_format == WAFER_FMT_BF16 ? launch_gemm<KIND_BF16, OUT_NARROW_RES>(ctx, args)
+                                     : launch_gemm<KIND_F16, OUT_NARROW_RES>(ctx, args);
 }
 
 extern "C" int wafer_hip_gemm_mfma_swiglu(wafer_hip_context *ctx, const void *lhs, const void *rhs_gu,
@@ -1457,8 +1417,8 @@ extern "C" int wafer_hip_gemm_mfma_swiglu(wafer_hip_context *ctx, const void *lh
   WAFER_TRY(check_hip(hipSetDevice(ctx->device), "hipSetDevice"));
   GemmArgs args{(const uint8_t *)lhs, (const uint8_t *)rhs_gu, dst, nullptr, nullptr, (int)m,
                 (int)(2 * features), (int)(k * 2), 0, 0};
-  return in_format == WAFER_FMT_BF16 ? launch_gemm<KIND_BF16, OUT_SWIGLU>(ctx->stream, args)
-                                     : launch_gemm<KIND_F16, OUT_SWIGLU>(ctx->stream, args);
+  return in_format == WAFER_FMT_BF16 ? launch_gemm<KIND_BF16, OUT_SWIGLU>(ctx, args)
+                                     : launch_gemm<KIND_F16, OUT_SWIGLU>(ctx, args);
 }
 
 extern "C" int wafer_hip_gemm_i8(wafer_hip_context *ctx, const int8_t *a, const int8_t *b,
@@ -1484,5 +1444,5 @@ extern "C" int wafer_hip_gemm_i8(wafer_hip_context *ctx, const int8_t *a, const 
   }
   if (rhs_orientation == WAFER_GEMM_NORMAL) WAFER_TRY(relayout_rhs(ctx, b, k, n, 1, &bt));
   GemmArgs args{(const uint8_t *)a, bt, y, acc_out, scale, (int)m, (int)n, (int)k, 0, 0};
-  return launch_gemm<KIND_I8, OUT_I8_DEQUANT>(ctx->stream, args);
+  return launch_gemm<KIND_I8, OUT_I8_DEQUANT>(ctx, args);
 }
