@@ -1,7 +1,8 @@
 """GPU tests of the MFMA GEMMs by row count: the weight-streaming kernel of few
 rows, at the edges of its 16-row tiles and of its column tiles, and with K
 that is not a whole 128-byte unit or leaves some of a workgroup's waves
-without one.
+without one; and the 4-wave tile kernel where its tiles do not divide the
+output.
 
 Against float64 on the same inputs: an f32 sum of K products in any order is
 within K 2^-24 sum |a| |b| of the exact one.  A 16-bit output adds half an ulp:
@@ -45,9 +46,14 @@ def _check(got, a, b, half_ulp):
 
 ROWS = [(1, 128, 4096, 3), (15, 130, 96, 2), (16, 16, 32, 3), (17, 4096, 160, 3), (31, 33, 8192, 2), (32, 8192, 96, 3),
         (33, 1000, 544, 2), (48, 10272, 64, 3), (63, 20, 2080, 3), (64, 12288, 128, 2), (64, 640, 1024, 3)]
+# tiles of the 4-wave kernel whose last row / column of tiles is shifted back
+# to the edge: 64x64, 64x128, 128x64, 128x128, 128x192 and 256x256, with n of
+# every alignment
+TILES = [(65, 64, 128, 3), (127, 72, 256, 2), (100, 16400, 128, 3), (129, 130, 192, 2), (300, 4100, 128, 3),
+         (300, 6145, 256, 2), (1000, 6148, 128, 3), (300, 28648, 64, 2), (300, 28656, 128, 3), (130, 60, 256, 3)]
 
 
-@pytest.mark.parametrize("m,n,k,fmt", ROWS)
+@pytest.mark.parametrize("m,n,k,fmt", ROWS + TILES)
 def test_gemm_rows_vs_float64(hip, B, m, n, k, fmt):
     print("[gemm rows]", m, n, k, fmt, flush=True)
     dt, half_ulp = (torch.bfloat16, 2.0 ** -8) if fmt == B.BF16 else (torch.float16, 2.0 ** -11)
@@ -83,7 +89,8 @@ def test_gemm_rows_vs_float64(hip, B, m, n, k, fmt):
         assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 100, 64), (16, 4096, 1024), (33, 1001, 4160), (64, 12288, 192)])
+@pytest.mark.parametrize("m,n,k", [(1, 100, 64), (16, 4096, 1024), (33, 1001, 4160), (64, 12288, 192),
+                                   (65, 100, 256), (300, 1000, 1024), (301, 4103, 128), (777, 6151, 128)])
 @pytest.mark.parametrize("rt", [False, True])
 def test_gemm_i8_rows_bit_exact(hip, B, m, n, k, rt):
     print("[gemm i8 rows]", m, n, k, rt, flush=True)
@@ -99,5 +106,8 @@ def test_gemm_i8_rows_bit_exact(hip, B, m, n, k, rt):
                 acc_out=acc, rhs_t=rt)
     assert np.array_equal(acc[:m * n].view(m, n).cpu().numpy(), acc_ref)
     yref = torch.from_numpy(acc_ref.astype(np.float32) * scale).to(torch.bfloat16)
+    assert torch.equal(y[:m * n].view(m, n).cpu(), yref)
+    hip.gemm_i8(torch.from_numpy(a).cuda(), torch.from_numpy(rhs).cuda(), torch.from_numpy(scale).cuda(), y.zero_(), m, k,
+                n, rhs_t=rt)  # without the accumulators: the staged stores
     assert torch.equal(y[:m * n].view(m, n).cpu(), yref)
     assert torch.all(acc[m * n:] == 0) and torch.all(y[m * n:] == 0)

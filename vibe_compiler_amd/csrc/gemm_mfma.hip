@@ -21,13 +21,13 @@
 // runs at a time form a 4x8 block of the output (whole rounds of 256 tiles),
 // or walk that XCD's own column strip in 4-row groups (other grids whose tile
 // rows divide by 4 and tile columns by 8), bounding the XCD's L2 working set.
-// Tiles are 256x256 when they fill the chip, 128x192 where that saves a round
-// of workgroups, else 128x128.  For 16-bit operands the 256x256, 256x224
-// (SwiGLU) and 128x192 tiles run on a 4-wave kernel instead (one wave per
-// SIMD, K slices moved by LDS DMA into a ring of 128 KiB), and long-K grids
-// of at most one round of 128x128 tiles split K over 4 workgroups of
-// 256x256 tiles with a fold launch.  Products of few rows go to the
-// weight-streaming kernel of gemm_skinny.hip.
+// For 16-bit operands, and int8 below 256x256 tiles, a 4-wave kernel (one wave
+// per SIMD, K slices moved by LDS DMA into a ring of 128 KiB) serves tiles
+// from 256x256 to 64x64, whichever the cost of their rounds says (pick_tile);
+// rows and columns that a tile does not divide end in a tile shifted back to
+// the edge.  Long-K grids of at most one round of 128x128 tiles may split K
+// over 4 workgroups of 256x256 tiles with a fold launch.  Products of few rows
+// go to the weight-streaming kernel of gemm_skinny.hip.
 //
 // int8 semantics (no reference implementation exists; the closed form on the
 // reference's conversion routes): acc = sum_k int32(a)*int32(b) exactly
@@ -115,8 +115,15 @@ __device__ inline void tile_coords(const GemmArgs &args, int bid, int &tm, int &
     tm = grp * 4 + w % 4;
     tn = xcd * sw + w / 4;
   } else {
-    tm = bid / tiles_n;
-    tn = bid % tiles_n;
+    // any other grid: XCD x takes a contiguous run of the tiles, walked in
+    // groups of up to 8 tile rows, column by column within a group, so that
+    // its rhs columns are read by one XCD
+    const int xcd = bid % 8, q = total / 8, r = total % 8;
+    const int idx = xcd * q + min(xcd, r) + bid / 8;
+    const int per_group = 8 * tiles_n, grp = idx / per_group, w = idx % per_group;
+    const int rows = min(8, tiles_m - 8 * grp);
+    tm = 8 * grp + w % rows;
+    tn = w / rows;
   }
 }
 
@@ -125,10 +132,12 @@ __device__ inline void tile_coords(const GemmArgs &args, int bid, int &tm, int &
 // this wave's LDS staging area of (BM/WM) x (output columns per wave) 16-bit
 // values, used after a barrier that retires every wave's main-loop LDS
 // traffic.
-template <int KIND, int BM, int BN, int OUT, bool TAIL, int WM, int WN, bool STAGE = true>
+// SHIFT: only rows from row_lo and (output) columns from col_lo on are
+// stored (the shifted last tiles of gemm_nt_dma4_kernel).
+template <int KIND, int BM, int BN, int OUT, bool TAIL, int WM, int WN, bool STAGE = true, bool SHIFT = false>
 __device__ __attribute__((always_inline)) inline void gemm_store(
     const GemmArgs &args, typename Acc<KIND>::T (&acc)[BM / WM / 32][BN / WN / 32], int m0, int n0,
-    char *stage) {
+    char *stage, int row_lo = 0, int col_lo = 0) {
   constexpr int WTM = BM / WM / 32, WTN = BN / WN / 32;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / WN, wn = wave % WN;
@@ -218,6 +227,7 @@ __device__ __attribute__((always_inline)) inline void gemm_store(
 #pragma unroll
       for (int q = 0; q < NQ; ++q) {
         const int idx = q * 64 + lane, row = idx / CPR, c = idx % CPR;
+        if (SHIFT && (m0 + wm * OR + row < row_lo || col0 + c * 8 < col_lo)) continue;
         u32x4 v = *(const u32x4 *)(stage + row * (CPR * 16) + (spos(row, c) << 4));
         if constexpr (OUT == OUT_NARROW_RES) {  // + the residual chunk at the same place
           const u32x4 rq =
@@ -268,6 +278,7 @@ __device__ __attribute__((always_inline)) inline void gemm_store(
           const uint16_t v = swiglu_pair<KIND>((float)acc[i][j][r], (float)acc[i][j][r + 1]);
           const int row = m0 + wm * (BM / WM) + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3) + hi;
           if (TAIL && !(col_ok && row < args.m)) continue;
+          if (SHIFT && (row < row_lo || feat < col_lo)) continue;
           ((uint16_t *)args.y)[(size_t)row * nf + feat] = v;
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -286,6 +297,7 @@ __device__ __attribute__((always_inline)) inline void gemm_store(
       for (int r = 0; r < 16; ++r) {
         const int row = m0 + wm * (BM / WM) + i * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
         if (TAIL && !(col_ok && row < args.m)) continue;
+        if (SHIFT && (row < row_lo || col < col_lo)) continue;
         const size_t o = (size_t)row * args.n + col;
         if (OUT == OUT_F32) {
           ((float *)args.y)[o] = (float)acc[i][j][r];
@@ -642,196 +654,9 @@ gemm_nt_kernel(GemmArgs args) {
   }
 }
 
-// Scheduling pins for one k-step of the 4-wave kernel: slot t holds one
-// MFMA, then (t+1) NR / NM - t NR / NM fragment reads and the same shares of
-// XL buffer loads and XW LDS writes.
-template <int T, int NM, int NR, int XL, int XW>
-__device__ __attribute__((always_inline)) inline void pin_slots() {
-  if constexpr (T < NM) {
-    constexpr int nr = ((T + 1) * NR) / NM - (T * NR) / NM;
-    constexpr int nl = ((T + 1) * XL) / NM - (T * XL) / NM;
-    constexpr int nw = ((T + 1) * XW) / NM - (T * XW) / NM;
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    if constexpr (nr > 0) __builtin_amdgcn_sched_group_barrier(0x100, nr, 0);
-    if constexpr (nl > 0) __builtin_amdgcn_sched_group_barrier(0x020, nl, 0);
-    if constexpr (nw > 0) __builtin_amdgcn_sched_group_barrier(0x200, nw, 0);
-    pin_slots<T + 1, NM, NR, XL, XW>();
-  }
-}
-
-// 4-wave tiles (2 x 2 waves, one per SIMD, the accumulators in AGPRs).
-// Against the 8-wave kernel each wave's sub-tile is twice as large, so the
-// LDS fragment reads per MFMA halve (256 x 256: 128 x 128 per wave).  K
-// slices of SB bytes are staged global -> VGPR -> LDS (16-byte buffer loads,
-// then ds_write_b128) instead of by LDS DMA, two register sets deep: the
-// loads for stage kt+2 are issued over the first half of stage kt's k-steps
-// and written to LDS in stage kt+1's second-to-last k-step, a stage and a
-// half of lead.  LDS rows are SB + 16 bytes (one 16-byte pad), so 16
-// consecutive rows read at one 16-byte chunk hit all 64 banks once and every
-// fragment address is a per-lane base plus an immediate.  K bytes a multiple
-// of 2 SB (an even number of stages); full tiles only.  16-bit operands (int8
-// keeps the 8-wave kernel: with the per-element dequant epilogue compiled in
-// this one spills the accumulators, and with the staged epilogue alone it is
-// bit-identical but no faster at 4096^3).  STAGE selects the LDS-staged
-// epilogue (else per-element stores).
-template <int KIND, int OUT, int BM, int BN, int SB, bool STAGE, int WM = 2, int WN = 2, bool SPLIT = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_rs_kernel(GemmArgs args) {
-  static_assert(WM * WN == 4, "four waves");
-  constexpr int PITCH = SB + 16, KS = SB / 32, CH = SB / 16, RPI = 64 / CH;
-  constexpr int WTM = BM / WM / 32, WTN = BN / WN / 32;
-  constexpr int A_INSTR = BM / RPI, B_INSTR = BN / RPI;  // RPI rows of SB bytes per wave instruction
-  constexpr int PER_WAVE = (A_INSTR + B_INSTR) / 4, NR = WTM + WTN, NM = WTM * WTN;
-  // k-steps carrying loads (the first half, else the first KS - 1, else the first) and loads per such k-step
-  constexpr int LK = PER_WAVE % (KS / 2) == 0 ? KS / 2 : PER_WAVE % (KS - 1) == 0 ? KS - 1 : 1;
-  constexpr int LPK = PER_WAVE / LK;
-  constexpr int WK = KS - 2;                             // the k-step that writes the older set to LDS
-  static_assert((A_INSTR + B_INSTR) % 4 == 0 && PER_WAVE % LK == 0, "loads split evenly");
-  constexpr int OC = OUT == OUT_SWIGLU ? BN / WN / 2 : BN / WN;
-  static_assert(!STAGE || 4 * (BM / WM) * OC * 2 <= 2 * (BM + BN) * PITCH, "staging fits in the ring");
-  __shared__ __align__(16) uint8_t lds[2 * (BM + BN) * PITCH];
-  // split-K: workgroup ids [s tiles, (s + 1) tiles) take split s
-  const int tiles = args.tiles_m * args.tiles_n;
-  const int split = SPLIT ? (int)blockIdx.x / tiles : 0;
-  int tm, tn;
-  tile_coords(args, (int)blockIdx.x - split * tiles, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wv / WN, wn = wv % WN;
-  const int l32 = lane & 31, g = lane >> 5;
-
-  typename Acc<KIND>::T acc[WTM][WTN];
-#pragma unroll
-  for (int i = 0; i < WTM; ++i)
-#pragma unroll
-    for (int j = 0; j < WTN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
-
-  // row stride kb; this workgroup's K slice starts at byte k0 and spans nkt stages
-  const int kb = args.kbytes;
-  const int kchunk = SPLIT ? kb / args.ksplit : kb;
-  const int k0 = split * kchunk, nkt = kchunk / SB;
-  const __amdgpu_buffer_rsrc_t ra =
-      __builtin_amdgcn_make_buffer_rsrc((void *)(args.a + (size_t)m0 * kb + k0), 0, BM * kb - k0, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rb =
-      __builtin_amdgcn_make_buffer_rsrc((void *)(args.bt + (size_t)n0 * kb + k0), 0, BN * kb - k0, 0x00020000);
-  // lane l moves 16-byte chunk l % CH of row l / CH of an RPI-row group
-  const int voff = (lane / CH) * kb + (lane % CH) * 16;
-  const int woff = (lane / CH) * PITCH + (lane % CH) * 16;
-
-  u32x4 stg[2][PER_WAVE];
-  auto gload = [&](int set, int kt, int q0, int q1) __attribute__((always_inline)) {
-    const int koff = min(kt, nkt - 1) * SB;  // past the last stage: a clamped copy, never used
-#pragma unroll
-    for (int q = q0; q < q1; ++q) {
-      const int ins = wv * PER_WAVE + q;
-      const bool is_a = ins < A_INSTR;
-      const int rel = is_a ? ins : ins - A_INSTR;
-      const int soff = __builtin_amdgcn_readfirstlane(rel * RPI * kb + koff);
-      stg[set][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(is_a ? ra : rb, voff, soff, 0));
-    }
-  };
-  auto lwrite = [&](int set, int buf) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < PER_WAVE; ++q) {
-      const int ins = wv * PER_WAVE + q;
-      const bool is_a = ins < A_INSTR;
-      const int rel = is_a ? ins : ins - A_INSTR;
-      *(u32x4 *)(lds + buf * (BM + BN) * PITCH + (is_a ? 0 : BM * PITCH) + rel * RPI * PITCH + woff) = stg[set][q];
-    }
-  };
-  // fragment rows wm*(BM/WM) + 32 i + l32 (A) and wn*(BN/WN) + 32 j + l32
-  // (Bt), 16-byte chunk 2 ks + g of the stage's slice
-  const int fa_base = (wm * (BM / WM) + l32) * PITCH + g * 16;
-  const int fb_base = (BM + wn * (BN / WN) + l32) * PITCH + g * 16;
-  u32x4 fa[2][WTM], fb[2][WTN];
-  // in the order the next k-step's MFMAs (row-major over i, j) consume them
-  auto read_frags = [&](int buf, int ks, int f) __attribute__((always_inline)) {
-    const uint8_t *base = lds + buf * (BM + BN) * PITCH + ks * 32;
-    fa[f][0] = *(const u32x4 *)(base + fa_base);
-#pragma unroll
-    for (int j = 0; j < WTN; ++j) fb[f][j] = *(const u32x4 *)(base + fb_base + j * 32 * PITCH);
-#pragma unroll
-    for (int i = 1; i < WTM; ++i) fa[f][i] = *(const u32x4 *)(base + fa_base + i * 32 * PITCH);
-  };
-  auto mfmas = [&](int f) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < WTM; ++i)
-#pragma unroll
-      for (int j = 0; j < WTN; ++j) acc[i][j] = mfma<KIND>(fa[f][i], fb[f][j], acc[i][j]);
-  };
-  // pins one k-step's order: NM slots of one MFMA followed by their share of
-  // the NR fragment reads, XL loads and XW LDS writes
-  auto pin = [&](auto XL, auto XW) __attribute__((always_inline)) {
-    pin_slots<0, NM, NR, decltype(XL)::value, decltype(XW)::value>();
-    __builtin_amdgcn_sched_barrier(0);
-  };
-
-  gload(0, 0, 0, PER_WAVE);
-  gload(1, 1, 0, PER_WAVE);
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_WAVE) : "memory");
-  lwrite(0, 0);
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  read_frags(0, 0, 0);
-
-  // Stage kt reads LDS buffer kt & 1.  Its first KS/2 k-steps issue the
-  // loads of stage kt+2 into register set kt & 1; k-step KS-2 writes set
-  // (kt+1) & 1 (stage kt+1, loaded during stage kt-1) to buffer (kt+1) & 1,
-  // which every wave finished reading before the previous stage barrier;
-  // the barrier sits before the last k-step.
-  auto stage = [&](int kt, auto P) __attribute__((always_inline)) {
-    constexpr int p = decltype(P)::value;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int cur = ks & 1;
-      if (ks < KS - 1) {
-        read_frags(p, ks + 1, cur ^ 1);
-        mfmas(cur);
-        if (ks < LK) gload(p, kt + 2, ks * LPK, (ks + 1) * LPK);
-        if (ks == WK) {
-          // set p^1 was issued a stage before set p: only set p may be in flight
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER_WAVE) : "memory");
-          lwrite(p ^ 1, p ^ 1);
-        }
-        constexpr int zero = 0;
-        (void)zero;
-        if (ks < LK && ks == WK) {
-          pin(std::integral_constant<int, LPK>{}, std::integral_constant<int, PER_WAVE>{});
-        } else if (ks < LK) {
-          pin(std::integral_constant<int, LPK>{}, std::integral_constant<int, 0>{});
-        } else if (ks == WK) {
-          pin(std::integral_constant<int, 0>{}, std::integral_constant<int, PER_WAVE>{});
-        } else {
-          pin(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-        }
-      } else {
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(p ^ 1, 0, cur ^ 1);
-        mfmas(cur);
-        pin(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{});
-      }
-    }
-  };
-  for (int kt = 0; kt < nkt; kt += 2) {
-    stage(kt, std::integral_constant<int, 0>{});
-    stage(kt + 1, std::integral_constant<int, 1>{});
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if constexpr (SPLIT) {
-    GemmArgs pa = args;
-    pa.y = args.part + (size_t)split * args.m * args.n;
-    gemm_store<KIND, BM, BN, OUT_F32, false, WM, WN, false>(pa, acc, m0, n0, nullptr);
-  } else {
-    gemm_store<KIND, BM, BN, OUT, false, WM, WN, STAGE>(args, acc, m0, n0, (char *)lds + wv * (BM / WM) * OC * 2);
-  }
-}
-
 // 4-wave tiles (one wave per SIMD, the accumulators in AGPRs) with the K
 // slices moved global -> LDS by buffer_load ... lds: no staging registers
-// and no LDS write instructions, which the register-staged kernel above
-// issues in bursts that fill the LDS data FIFO.  Stages of SB bytes of K per
+// and no LDS write instructions.  Stages of SB bytes of K per
 // row (SB / 32 MFMA k-steps) in a ring of 128 KiB (two stages of 256 + 256
 // rows at SB = 128, three of 128 + 192 rows).  One DMA instruction fills
 // 1024 / SB rows: lane l writes chunk position l % (SB / 16) of its row, so
@@ -846,8 +671,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // MFMA slots of two k-steps (a burst of them fills the texture address
 // FIFO): the first half in the last k-step of the stage whose slot it
 // refills, the second in the next stage's first k-step.  K bytes a multiple
-// of SB; full tiles only.
-template <int KIND, int OUT, int BM, int BN, int SB = 64, int WM = 2, int WN = 2, bool SPLIT = false>
+// of SB.  SHIFT serves m >= BM and n >= BN that the tile does not divide: the
+// last tile row (column) starts at m - BM (n - BN), so every load is in range
+// and the loop is the full tile's, and it stores only the rows (columns) that
+// the tile before it does not.
+//
+// Measured on cold weights against the 8-wave kernel's 128- and 256-row tiles
+// that served these shapes (us, bits unchanged): 128 x 4096, K 4096 36.8 ->
+// 21.0 (64x64), 300 x 6144 37.5 -> 31.3 (64x128), 300 x 4096 32.6 -> 27.7
+// (128x64), 777 x 6144 69.8 -> 54.6 (128x192), SwiGLU 128 x 28672 119.4 -> 59.4
+// (128x128), SwiGLU 777 x 28672 243.6 -> 215.1 (256x256).
+template <int KIND, int OUT, int BM, int BN, int SB = 64, int WM = 2, int WN = 2, bool SPLIT = false,
+          bool SHIFT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_nt_dma4_kernel(GemmArgs args) {
   static_assert(WM * WN == 4, "four waves");
   static_assert(SB == 64 || SB == 128, "64- or 128-byte stages");
@@ -870,7 +705,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int split = SPLIT ? (int)blockIdx.x / tiles : 0;
   int tm, tn;
   tile_coords(args, (int)blockIdx.x - split * tiles, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
+  // SHIFT: the last tile row / column starts early enough to end at m / n,
+  // and stores only what the tile before it does not
+  const int row_lo = tm * BM, col_lo = tn * BN;
+  const int m0 = SHIFT ? min(row_lo, args.m - BM) : row_lo, n0 = SHIFT ? min(col_lo, args.n - BN) : col_lo;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wv / WN, wn = wv % WN;
@@ -1002,9 +840,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   if constexpr (SPLIT) {
     GemmArgs pa = args;
     pa.y = args.part + (size_t)split * args.m * args.n;
-    gemm_store<KIND, BM, BN, OUT_F32, false, WM, WN, false>(pa, acc, m0, n0, nullptr);
+    gemm_store<KIND, BM, BN, OUT_F32, false, WM, WN, false, SHIFT>(pa, acc, m0, n0, nullptr, row_lo, col_lo);
   } else {
-    gemm_store<KIND, BM, BN, OUT, false, WM, WN, true>(args, acc, m0, n0, (char *)lds + wv * (BM / WM) * OC * 2);
+    gemm_store<KIND, BM, BN, OUT, false, WM, WN, true, SHIFT>(args, acc, m0, n0,
+                                                              (char *)lds + wv * (BM / WM) * OC * 2, row_lo,
+                                                              OUT == OUT_SWIGLU ? col_lo / 2 : col_lo);
   }
 }
 
@@ -1146,51 +986,149 @@ __global__ __launch_bounds__(256) void transpose_any_kernel(const T *__restrict_
     if (n0 + i < N && k0 + tx < K) dst[(size_t)(n0 + i) * K + k0 + tx] = tile[tx][i];
 }
 
-template <int KIND, int OUT, int SB>
-int launch_gemm_tiles(hipStream_t st, GemmArgs args);
+// ---- which kernel and tile serve a product
 
-template <int KIND, int OUT, int SB>
-int launch_gemm_sb(hipStream_t st, GemmArgs args) {
-  if constexpr (OUT != OUT_SWIGLU) {
-    return launch_gemm_tiles<KIND, OUT, SB>(st, args);
-  } else {
-    // 256x224 tiles (4 x 1 waves of 64 x 224, LDS-DMA staging) where their
-    // rounds of 256 workgroups take less time than those of 256x256 tiles
-    // (gate/up at n 28672: 512 tiles in two rounds of 7/8 the work, against
-    // 448 tiles whose second round is three quarters full; 211 against
-    // 217 us register-staged in the decoder layer)
-    if constexpr (SB == 128) {
-      if (args.m % 256 == 0 && args.n % 224 == 0 && args.kbytes % 256 == 0) {
-        const long t224 = (long)(args.m / 256) * (args.n / 224), t256 = (long)(args.m / 256) * ((args.n + 255) / 256);
-        if (7 * ((t224 + 255) / 256) < 8 * ((t256 + 255) / 256)) {
-          args.tiles_m = args.m / 256;
-          args.tiles_n = args.n / 224;
-          hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, 256, 224, 128, 4, 1>),
-                             dim3(args.tiles_m * args.tiles_n), dim3(256), 0, st, args);
-          return launch_status("gemm_nt_dma4_kernel");
-        }
-      }
+// Time of one round of tiles (one workgroup per CU) on the 4-wave LDS-DMA
+// kernel: ns per 128-byte K stage and ns per tile besides, fitted to bf16
+// runs at K 4096 with the grid in one round (84 us for 256x256, 49 for 128x192,
+// 36 for 128x128, 27 for 128x64, 28.5 for 64x128, 20.5 for 64x64).  A smaller
+// tile moves more operand bytes and reads more fragments per FLOP; it is the
+// faster one where the larger leaves CUs without a tile or rows unused.
+struct TileCost { int bm, bn, stage_ns, tile_ns; };
+constexpr TileCost TILES[] = {{256, 256, 1250, 6000}, {256, 224, 1200, 6000}, {128, 192, 690, 4000},
+                              {128, 128, 500, 3500},  {128, 64, 410, 2500},   {64, 128, 425, 2500},
+                              {64, 64, 285, 2000}};
+
+// The tile for m x n outputs (-1: none, the product is narrower than every
+// tile).  256x224 tiles serve SwiGLU products that they divide.  Examples at
+// K 4096: (1024, 6144) 128x192, (1024, 4096) 128x128, (300, 4096) 128x64,
+// (300, 6144) 64x128, (128, 4096) 64x64.
+int pick_tile(int m, int n, int kbytes, bool swiglu, int cus, long *ns) {
+  int best = -1;
+  for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
+    const TileCost &t = TILES[i];
+    if (m < t.bm || n < t.bn) continue;
+    if (t.bn == 224 && !(swiglu && m % 256 == 0 && n % 224 == 0)) continue;
+    const long tiles = (long)((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+    const long cost = ((tiles + cus - 1) / cus) * ((long)t.stage_ns * (kbytes / 128) + t.tile_ns);
+    if (best < 0 || cost < *ns) {
+      best = i;
+      *ns = cost;
     }
-    args.tiles_m = (args.m + 255) / 256;
-    args.tiles_n = (args.n + 255) / 256;
-    const dim3 grid(args.tiles_m * args.tiles_n);
-    if (args.m % 256 == 0 && args.n % 256 == 0 && args.kbytes % 256 == 0)
-      hipLaunchKernelGGL((gemm_nt_rs_kernel<KIND, OUT, 256, 256, 128, false>), grid, dim3(256), 0, st, args);
-    else if (args.m % 256 == 0 && args.n % 256 == 0)
-      hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, false, SB>), grid, dim3(512), 0, st, args);
-    else
-      hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, true, SB>), grid, dim3(512), 0, st, args);
-    return launch_status("gemm_nt_kernel");
   }
+  return best;
 }
 
+template <int KIND, int OUT, int BM, int BN, int WM = 2, int WN = 2>
+int launch_dma4(hipStream_t st, GemmArgs args) {
+  args.tiles_m = (args.m + BM - 1) / BM;
+  args.tiles_n = (args.n + BN - 1) / BN;
+  const dim3 grid(args.tiles_m * args.tiles_n);
+  if constexpr (BM * BN >= 128 * 128) {
+    if (args.m % BM == 0 && args.n % BN == 0) {
+      hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, BM, BN, 128, WM, WN>), grid, dim3(256), 0, st, args);
+      return launch_status("gemm_nt_dma4_kernel");
+    }
+  }
+  if constexpr (BN != 224)
+    hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, BM, BN, 128, WM, WN, false, true>), grid, dim3(256), 0, st,
+                       args);
+  return launch_status("gemm_nt_dma4_kernel");
+}
+
+// The 8-wave kernel: 64-byte K stages, products narrower than 64 columns,
+// int8 on 256x256 tiles, and 128x128 tiles over a very long K.
 template <int KIND, int OUT, int SB>
-int launch_gemm_tiles(hipStream_t st, GemmArgs args) {
-  // split-K planned by the entry (plan_split, partial area in args.part), on
-  // the LDS-DMA kernel (the decoder layer's down projection: 106 against
-  // 115 us register-staged)
-  if constexpr (KIND != KIND_I8 && SB == 128) {
-    if (args.ksplit > 1) {
+int launch_wave8(hipStream_t st, GemmArgs args) {
+  const int side = OUT == OUT_SWIGLU || (args.m % 256 == 0 && args.n % 256 == 0 &&
+                                         (long)(args.m / 256) * (args.n / 256) >= 192) ? 256 : 128;
+  args.tiles_m = (args.m + side - 1) / side;
+  args.tiles_n = (args.n + side - 1) / side;
+  const dim3 grid(args.tiles_m * args.tiles_n);
+  const bool full = args.m % side == 0 && args.n % side == 0;
+  if (side == 256 && full) {
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, false, SB>), grid, dim3(512), 0, st, args);
+  } else if constexpr (OUT == OUT_SWIGLU) {
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, true, SB>), grid, dim3(512), 0, st, args);
+  } else if (full) {
+    // 4 x 2 waves (each 32 x 64) measured 2-3 % faster than 2 x 4 on 128x128
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, false, SB, 4, 2>), grid, dim3(512), 0, st, args);
+  } else {
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, true, SB, 4, 2>), grid, dim3(512), 0, st, args);
+  }
+  return launch_status("gemm_nt_kernel");
+}
+
+template <int KIND, int OUT>
+int launch_tile(hipStream_t st, GemmArgs args, int tile) {
+  const int bm = TILES[tile].bm, bn = TILES[tile].bn;
+  if constexpr (KIND == KIND_I8) {
+    // whole 256x256 tiles keep 8 waves (int8 4096^3: 65.3 us against 68.5)
+    if (bm == 256) {
+      if (args.m % 256 == 0 && args.n % 256 == 0) return launch_wave8<KIND, OUT, 128>(st, args);
+      return launch_dma4<KIND, OUT, 128, 128>(st, args);
+    }
+  } else {
+    if (bm == 256 && bn == 256) return launch_dma4<KIND, OUT, 256, 256>(st, args);
+  }
+  if constexpr (OUT == OUT_SWIGLU) {
+    if (bn == 224) return launch_dma4<KIND, OUT, 256, 224, 4, 1>(st, args);
+  }
+  if (bn == 192) return launch_dma4<KIND, OUT, 128, 192>(st, args);
+  // past K 12288 the 8-wave kernel serves 128x128 tiles (777 x 4096, K 14336:
+  // 127 us against 145; K 11008: 101 against 102; 900 x 4096, K 8192: 83
+  // against 72)
+  if (bm == 128 && bn == 128)
+    return args.kbytes >= 24576 ? launch_wave8<KIND, OUT, 128>(st, args)
+                                : launch_dma4<KIND, OUT, 128, 128>(st, args);
+  if (bm == 128) return launch_dma4<KIND, OUT, 128, 64, 4, 1>(st, args);
+  if (bn == 128) return launch_dma4<KIND, OUT, 64, 128>(st, args);
+  return launch_dma4<KIND, OUT, 64, 64>(st, args);
+}
+
+// Split-K plan for 16-bit GEMMs whose 128x128 grid is at most one round of
+// workgroups and whose K is long: 256x256 tiles on the 4-wave kernel (half
+// the operand bytes per FLOP of 128x128 tiles), each tile's K split over
+// ksplit workgroups so that the grid still fills the CUs, plus a fold
+// launch, where no unsplit tile takes less time (the partial tiles are
+// written and read again at about 5 TB/s).  Returns 1 (no split) otherwise.
+// The decoder layer's down projection (1024 x 4096, K 14336, with the
+// residual): 113.3 us + 14.2 us fold against 136.1 us on 128x128 tiles;
+// 256x128 tiles with two splits (32 MiB of partials instead of 64) measured
+// 138.3 + 9.3 us.  At 256 x 4096, 64x64 tiles: 74 us against 98 split.
+int plan_split(int m, int n, int kbytes, int cus) {
+  if (m % 256 != 0 || n % 256 != 0 || kbytes < 16384) return 1;
+  const long t2 = (long)(m / 256) * (n / 256), t128 = (long)(m / 128) * (n / 128);
+  if (t128 > cus) return 1;
+  long whole = 0;
+  pick_tile(m, n, kbytes, false, cus, &whole);
+  for (int s = 4; s >= 2; --s)
+    if (t2 * s <= cus && kbytes % (256 * s) == 0) {  // whole pairs of 128-byte stages per split
+      const long split = 1250L * (kbytes / s / 128) + 6000 + 2500 + (long)m * n * (8 * s + 4) / 5000;
+      return split < whole ? s : 1;
+    }
+  return 1;
+}
+
+// Sets up args.ksplit / args.part for a 16-bit GEMM (growing the context's
+// partial-tile area when a split is planned).
+int prepare_split(wafer_hip_context *ctx, GemmArgs &args) {
+  if (gemm_is_skinny(args.m)) return WAFER_HIP_OK;
+  const int s = plan_split(args.m, args.n, args.kbytes, ctx->cu_count > 0 ? ctx->cu_count : 256);
+  if (s < 2) return WAFER_HIP_OK;
+  WAFER_TRY(ensure_workspace(ctx, &ctx->partials, &ctx->partials_bytes, (size_t)s * args.m * args.n * sizeof(float)));
+  args.ksplit = s;
+  args.part = (float *)ctx->partials;
+  return WAFER_HIP_OK;
+}
+
+template <int KIND, int OUT>
+int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
+  const hipStream_t st = ctx->stream;
+  const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  if (gemm_is_skinny(args.m)) return launch_gemm_skinny<KIND, OUT>(st, args, cus);
+  if constexpr (KIND != KIND_I8 && OUT != OUT_SWIGLU) {
+    if (args.ksplit > 1) {  // planned by the entry (prepare_split)
       args.tiles_m = args.m / 256;
       args.tiles_n = args.n / 256;
       hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT_F32, 256, 256, 128, 2, 2, true>),
@@ -1203,110 +1141,10 @@ int launch_gemm_tiles(hipStream_t st, GemmArgs args) {
       return launch_status("gemm_fold_kernel");
     }
   }
-  // 256x256 tiles only where they divide the output and still fill the chip
-  if (args.m % 256 == 0 && args.n % 256 == 0 && (args.m / 256) * (args.n / 256) >= 192) {
-    args.tiles_m = args.m / 256;
-    args.tiles_n = args.n / 256;
-    // 16-bit operands with an even number of 128-byte K stages: 4 waves,
-    // register-staged (int8 keeps 8 waves: its 4-wave dequant epilogue
-    // spills; a residual keeps the 8-wave kernel's staged epilogue)
-    if constexpr (KIND != KIND_I8 && OUT != OUT_NARROW_RES) {
-      if (args.kbytes % 128 == 0) {
-        // LDS-DMA staging (4096^3: 107 against 111 us register-staged)
-        hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, 256, 256, 128>), dim3(args.tiles_m * args.tiles_n),
-                           dim3(256), 0, st, args);
-        return launch_status("gemm_nt_dma4_kernel");
-      }
-    }
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, false, SB>), dim3(args.tiles_m * args.tiles_n),
-                       dim3(512), 0, st, args);
-    return launch_status("gemm_nt_kernel");
-  }
-  // 128x192 tiles where they need fewer rounds of 256 workgroups for 1.5x
-  // the work per tile (QKV at M = 1024: 256 tiles against 384 of 128x128)
-  // (128-byte K stages only: 64-byte stages would not split 320 rows of DMA
-  // evenly over 8 waves)
-  const long t128 = (long)((args.m + 127) / 128) * ((args.n + 127) / 128);
-  if (SB == 128 && args.m % 128 == 0 && args.n % 192 == 0) {
-    const long t192 = (long)(args.m / 128) * (args.n / 192);
-    if (3 * ((t192 + 255) / 256) < 2 * ((t128 + 255) / 256)) {
-      args.tiles_m = args.m / 128;
-      args.tiles_n = args.n / 192;
-      if constexpr (SB == 128) {
-        // 16-bit operands, plain outputs: the 4-wave kernel (QKV at M = 1024:
-        // 53.3 against 55.4 us); a residual keeps the 8-wave kernel's staged
-        // epilogue
-        if constexpr (KIND != KIND_I8 && OUT != OUT_NARROW_RES) {
-          if (args.kbytes % 128 == 0) {
-            // LDS-DMA staging, three stages (QKV at M = 1024 in the decoder
-            // layer: 52.5 against 59.4 us register-staged)
-            hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, 128, 192, 128>), dim3(args.tiles_m * args.tiles_n),
-                               dim3(256), 0, st, args);
-            return launch_status("gemm_nt_dma4_kernel");
-          }
-        }
-        hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 192, OUT, false, SB, 4, 2>),
-                           dim3(args.tiles_m * args.tiles_n), dim3(512), 0, st, args);
-        return launch_status("gemm_nt_kernel");
-      }
-    }
-  }
-  args.tiles_m = (args.m + 127) / 128;
-  args.tiles_n = (args.n + 127) / 128;
-  const dim3 grid(args.tiles_m * args.tiles_n);
-  // full 16-bit tiles with plain outputs: the 4-wave LDS-DMA kernel, each
-  // wave 64x64 (the decoder layer's O projection, 1024 x 4096 x 4096: 36.0
-  // against 41.4 us on the 8-wave register-staged kernel)
-  if constexpr (KIND != KIND_I8 && OUT != OUT_NARROW_RES && SB == 128) {
-    if (args.m % 128 == 0 && args.n % 128 == 0) {
-      hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, 128, 128, 128>), grid, dim3(256), 0, st, args);
-      return launch_status("gemm_nt_dma4_kernel");
-    }
-  }
-  // ragged, int8, residual or 64-byte-stage GEMMs: 4 x 2 waves (each 32 x 64)
-  // measured 2-3 % faster than 2 x 4 on 128x128 tiles
-  if (args.m % 128 == 0 && args.n % 128 == 0)
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, false, SB, 4, 2>), grid, dim3(512), 0, st, args);
-  else
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, true, SB, 4, 2>), grid, dim3(512), 0, st, args);
-  return launch_status("gemm_nt_kernel");
-}
-
-// Split-K plan for 16-bit GEMMs whose 128x128 grid is at most one round of
-// workgroups and whose K is long: 256x256 tiles on the 4-wave kernel (half
-// the operand bytes per FLOP of 128x128 tiles), each tile's K split over
-// ksplit workgroups so that the grid still fills the CUs, plus a fold
-// launch.  Returns 1 (no split) otherwise.  The decoder layer's down
-// projection (1024 x 4096, K 14336, with the residual): 113.3 us + 14.2 us
-// fold against 136.1 us on 128x128 tiles; 256x128 tiles with two splits
-// (32 MiB of partials instead of 64) measured 138.3 + 9.3 us.
-int plan_split(int m, int n, int kbytes, int cus) {
-  if (m % 256 != 0 || n % 256 != 0 || kbytes < 16384) return 1;
-  const long t2 = (long)(m / 256) * (n / 256), t128 = (long)(m / 128) * (n / 128);
-  if (t128 > cus) return 1;
-  for (int s = 4; s >= 2; --s)
-    if (t2 * s <= cus && kbytes % (256 * s) == 0) return s;  // whole pairs of 128-byte stages per split
-  return 1;
-}
-
-// Sets up args.ksplit / args.part for a 16-bit GEMM (growing the context's
-// partial-tile area when a split is planned).
-int prepare_split(wafer_hip_context *ctx, GemmArgs &args) {
-  const int s = plan_split(args.m, args.n, args.kbytes, ctx->cu_count > 0 ? ctx->cu_count : 256);
-  if (s < 2) return WAFER_HIP_OK;
-  WAFER_TRY(ensure_workspace(ctx, &ctx->partials, &ctx->partials_bytes, (size_t)s * args.m * args.n * sizeof(float)));
-  args.ksplit = s;
-  args.part = (float *)ctx->partials;
-  return WAFER_HIP_OK;
-}
-
-template <int KIND, int OUT>
-int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
-  const hipStream_t st = ctx->stream;
-  if (gemm_is_skinny(args.m))
-    return launch_gemm_skinny<KIND, OUT>(st, args, ctx->cu_count > 0 ? ctx->cu_count : 256);
-  // 128-byte K stages where K allows (half the stage barriers per FLOP)
-  return args.kbytes % 128 == 0 ? launch_gemm_sb<KIND, OUT, 128>(st, args) : launch_gemm_sb<KIND, OUT, 64>(st, args);
+  if (args.kbytes % 128 != 0) return launch_wave8<KIND, OUT, 64>(st, args);
+  long ns = 0;
+  const int tile = pick_tile(args.m, args.n, args.kbytes, OUT == OUT_SWIGLU, cus, &ns);
+  return tile < 0 ? launch_wave8<KIND, OUT, 128>(st, args) : launch_tile<KIND, OUT>(st, args, tile);
 }
 
 int relayout_rhs(wafer_hip_context *ctx, const void *rhs, uint32_t k, uint32_t n, int esize,
