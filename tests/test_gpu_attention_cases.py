@@ -435,3 +435,71 @@ def test_hugely_negative_visible_scores_keep_their_maximum(hip, oracle, fmt, D):
     best = int(np.argmax(bias[0, 0, 0]))
     assert np.array_equal(got[0, 0], np.broadcast_to(v[0, 0, best], (Sq, D)))
     assert np.array_equal(got, oracle.attention_prefill_ex(q, k, v, 0.125, bias=bias, fmt=fmt))
+
+
+def _padding(rng, Bn, L):
+    """Per-sequence key masks: a leading gap, a hole, a short tail, one key."""
+    keep = np.ones((Bn, 1, 1, L), np.uint8)
+    keep[0, ..., : L // 3] = 0
+    keep[0, ..., L - 1:] = 0
+    if Bn > 1:
+        keep[1] = rng.integers(0, 2, (1, 1, L)) * rng.integers(1, 256, (1, 1, L))  # any nonzero byte shows a key
+    if Bn > 2:
+        keep[2] = 0
+        keep[2, ..., L // 2] = 1
+    return keep
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Sq,L", [(1, 1), (3, 2), (5, 3), (65, 63), (64, 64), (130, 65), (257, 193), (70, 1031),
+                                  (640, 640), (64, 65600)])
+def test_boolean_masks(hip, oracle, D, Sq, L):
+    """Boolean masks that are the same for every query (held as one bit per
+    key up to 65536 keys) and masks per query, with a window on top, at key
+    counts around the 64-key blocks and below the four keys of one load,
+    against a float64 softmax under the attention policy; rows that see no
+    key are exactly +0, and a mask of ones is no mask, bit for bit."""
+    say("boolean masks", D, Sq, L)
+    rng = np.random.default_rng(Sq * 7 + L + D)
+    Bn, Hq, Hkv = (1, 1, 1) if L > 4096 else (3, 4, 2)
+    q, k, v = inputs(oracle, rng, F16, Hq, Hkv, Sq, L, D, Bn)
+    scale = 1.0 / math.sqrt(D)
+    tq, tk, tv = (torch.from_numpy(oracle.to_float(F16, x).reshape(x.shape)).double().cuda() for x in (q, k, v))
+    tk, tv = (x.repeat_interleave(Hq // Hkv, dim=1) for x in (tk, tv))
+    scores = (tq.cpu() @ tk.cpu().transpose(2, 3)).cuda() * scale  # the batched product on the CPU
+    per_query = rng.integers(0, 2, (Bn, Hq, Sq, L)).astype(np.uint8)
+    per_query[:, :, Sq // 2] = 0
+    cases = [dict(keep=_padding(rng, Bn, L)), dict(keep=per_query),
+             dict(keep=_padding(rng, Bn, L), causal=True, diagonal=L - Sq, window=max(1, L // 2))]
+    for kw in cases:
+        vis = torch.from_numpy(np.broadcast_to(kw["keep"] != 0, (Bn, Hq, Sq, L)).copy()).cuda()
+        if kw.get("causal"):
+            vis &= torch.from_numpy(band(Sq, L, kw["diagonal"], kw["window"])).cuda()
+        p = torch.softmax(scores.masked_fill(~vis, float("-inf")), dim=-1).nan_to_num(0.0)
+        ref = (p.cpu() @ tv.cpu()).numpy()
+        got = tof(oracle, F16, run_masked(hip, F16, q, k, v, scale, **kw))
+        none = ~vis.any(dim=-1).cpu().numpy()
+        assert not got[none].any()
+        if (~none).any():
+            attention_gate(got, ref.astype(np.float32), what=f"keep {list(kw)}")
+    ones = run_masked(hip, F16, q, k, v, scale, keep=np.ones((1, 1, 1, L), np.uint8))
+    assert np.array_equal(ones, run_masked(hip, F16, q, k, v, scale))
+
+
+@pytest.mark.parametrize("L", [1, 2, 65, 191])
+def test_additive_mask_tails(hip, oracle, L):
+    """An additive mask per query whose rows end inside a 64-key block, with
+    -inf and the lowest finite float among its values."""
+    say("additive tails", L)
+    rng = np.random.default_rng(L)
+    for D in (64, 128):
+        q, k, v = inputs(oracle, rng, BF16, 2, 1, 70, L, D)
+        bias = rng.standard_normal((1, 2, 70, L)).astype(np.float32)
+        bias[..., 3, :] = np.finfo(np.float32).min
+        bias[..., 4, :] = -np.inf
+        bias[..., 5, : L // 2] = -np.inf
+        kw = dict(bias=bias)
+        ref = oracle.attention_prefill_ex(q, k, v, 0.125, fmt=BF16, **kw)
+        got = run_masked(hip, BF16, q, k, v, 0.125, **kw)
+        attention_gate(tof(oracle, BF16, got), tof(oracle, BF16, ref), what="additive tail")
+        assert not got[:, :, 4].any()

@@ -37,8 +37,17 @@
 //      then.  P <= 2^8 and its narrowing point differs from the
 //      reference's with the same relative bound;
 //    - MASK_CAUSAL masks by position only (no mask operands, no rounding);
-//      MASK_GENERAL evaluates the whole score region per element in the
-//      natural-log domain and hands u = t*log2(e) to the exponentials.
+//      MASK_SELECT also takes a window and a boolean mask, as one bit per
+//      score (nothing is done to a block that the wave sees whole); MASK_GENERAL
+//      evaluates the whole score region per element in the natural-log domain
+//      and hands u = t*log2(e) to the exponentials.  What bounded these was
+//      mask loads: one byte or float per score, each waited for.  A boolean mask
+//      that is the same for every query (a padding mask) is now read once into
+//      LDS bits, and its first and last visible key bound the key blocks
+//      walked; other masks are loaded four keys at a time, an iteration ahead.
+//      Measured (us): padding mask, 4 x 8 heads x 1031, head_dim 64: 164 -> 28;
+//      window of 256, 8 heads x 1024, head_dim 64: 32.9 -> 8.2; additive mask,
+//      the same shape: 125 -> 34.5, and 32 heads x 1000, head_dim 128: 152 -> 84.
 //  * fa_small<T> (head_dim <= 64 other than 64): one thread per query row,
 //    K / V blocks of 64 keys staged as f32 in LDS, the reference's block
 //    update evaluated per row in its own order (dot products as fma chains
@@ -53,6 +62,7 @@ namespace {
 constexpr int QB = 64;        // queries per query block (two 32-query wave tiles)
 constexpr int BK = 64;        // keys per KV block
 constexpr int THREADS = 256;  // 4 waves: (tile, key half)
+constexpr int KEEP_BLOCKS = 1024;  // key blocks of a per-key boolean mask held as LDS bits (8 KiB)
 constexpr float RESCALE_LOG2 = 8.0f;
 constexpr float RESCALE_BOUND = 256.0f;
 // "no reference yet": the lowest finite float, so exp2(u - NOREF) is +inf
@@ -63,7 +73,7 @@ constexpr float RESCALE_BOUND = 256.0f;
 constexpr float NOREF = -0x1.fffffep127f;
 constexpr float LOG2E = 0x1.715476p+0f;
 
-enum { MASK_CAUSAL = 1, MASK_GENERAL = 2 };
+enum { MASK_CAUSAL = 1, MASK_GENERAL = 2, MASK_SELECT = 3 };
 constexpr uint32_t F_CAUSAL = WAFER_HIP_ATT_CAUSAL, F_WINDOW = WAFER_HIP_ATT_WINDOW,
                    F_ROUND_SCALED = WAFER_HIP_ATT_ROUND_SCALED, F_ROUND_BIASED = WAFER_HIP_ATT_ROUND_BIASED;
 
@@ -74,6 +84,7 @@ struct FaArgs {
   float c;      // scale * log2(e)
   float scale;
   int bh_count, n_qblocks;
+  int single;  // one query block per workgroup instead of a late and an early one
   uint32_t flags;
   int diag;     // CAUSAL: key j visible to query i only if j <= i + diag
   int lo_off;   // WINDOW: and j >= i + lo_off (lo_off = diag - window + 1)
@@ -126,20 +137,25 @@ __device__ inline float xor32_sum(float x) {
 
 // One score through the score region and the masks: visible -> u = t*log2(e)
 // (a finite t whose u overflows is clamped to the lowest finite float),
-// invisible -> -inf, whatever t is (an invisible key is excluded).
+// invisible -> -inf, whatever t is (an invisible key is excluded).  Selects
+// only: a branch here would be taken 32 times per block.
 template <typename T>
-__device__ inline float general_score(float s, float scale, uint32_t flags, const float *brow,
-                                      const uint8_t *krow, int key, bool vis) {
-  float t = s * scale;
-  if (flags & F_ROUND_SCALED) t = round_to<T>(t);
-  if (vis && brow) {
-    t = t + brow[key];
-    if (flags & F_ROUND_BIASED) t = round_to<T>(t);
-  }
-  if (vis && krow) vis = krow[key] != 0;
-  if (!vis || t == -__builtin_inff()) return -__builtin_inff();
-  const float u = t * LOG2E;
-  return u == u ? fmaxf(u, NOREF) : u;  // NaN passes through
+__device__ inline float general_score(float s, float scale, bool round_scaled, bool round_biased, float bias, bool vis) {
+  const float t0 = s * scale, t0r = round_to<T>(t0);
+  const float t1 = (round_scaled ? t0r : t0) + bias, t1r = round_to<T>(t1);
+  const float t = round_biased ? t1r : t1;
+  const float u = t * LOG2E, c = fmaxf(u, NOREF);
+  const float v = u == u ? c : u;  // NaN passes through
+  return vis && t != -__builtin_inff() ? v : -__builtin_inff();
+}
+
+// Mask bytes of keys key .. key + 3 of a row of n >= 4 (the bytes of keys at
+// or past n are not defined, and no byte outside the row is read).
+__device__ inline uint32_t keep_word(const uint8_t *row, int key, int n) {
+  const int at = min(key, n - 4), sh = 8 * (key - at);
+  uint32_t w;
+  __builtin_memcpy(&w, row + at, 4);
+  return sh < 32 ? w >> sh : 0;
 }
 
 // LDS swizzles (16-byte chunk index XOR): K rows are read 32 rows x one
@@ -153,8 +169,16 @@ __device__ inline int swz_v(int row) {
   return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1);
 }
 
+// Waves per SIMD: at head_dim 64 two workgroups fit a CU (256 registers per
+// wave, a few of them spilled outside the pipelined iteration), and one's
+// matrix work covers the other's softmax (4 x 8 heads x 1031: 34.5 -> 26.7 us);
+// the score region's mask operands do not fit that way (34.5 against 52.7 us at
+// 8 heads x 1024 with an additive mask).
+constexpr int fa_waves(int d, int mask) { return d == 64 && mask != MASK_GENERAL ? 2 : 1; }
+
 template <typename T, int D, int MASK>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1))) void fa_fwd(const FaArgs a) {
+__global__ __launch_bounds__(THREADS)
+__attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void fa_fwd(const FaArgs a) {
   constexpr int ROWB = 2 * D;            // bytes per K / V row
   constexpr int CH = ROWB / 16;          // 16-byte chunks per row
   constexpr int RPI = 64 / CH;           // rows per 1 KiB DMA instruction
@@ -167,6 +191,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
   // read and waits for the moves only at the iteration's barrier
   __shared__ __align__(1024) char sk0[2 * BLK], sk1[2 * BLK], sv0[2 * BLK], sv1[2 * BLK];
   __shared__ float sml[4][2][64];
+  // a boolean mask that is the same for every query, one bit per key
+  __shared__ uint32_t skeep[MASK == MASK_CAUSAL ? 1 : KEEP_BLOCKS * 2];
 
   const int bid = blockIdx.x;
   const int pair = bid / a.bh_count;
@@ -183,13 +209,55 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
   const int tile = wave & 1, half = wave >> 1;
   const int l32 = lane & 31, g = lane >> 5;
 
+  // A boolean mask that is the same for every query (a padding mask) is read
+  // once, into one LDS bit per key; its first and last visible key bound the
+  // key blocks walked.
+  int seen_lo = 0, seen_hi = a.kv_len - 1;
+  const bool row_mask = MASK != MASK_CAUSAL && a.keep && a.keep_sq == 0 && a.kv_len <= KEEP_BLOCKS * BK;
+  if (MASK != MASK_CAUSAL && row_mask) {
+    const uint8_t *row = a.keep + b * a.keep_sb + h * a.keep_sh;
+    int lo = a.kv_len, hi = -1;
+    for (int k0 = 0; k0 < a.kv_len; k0 += 4 * THREADS) {
+      uint8_t v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = k0 + i * THREADS + tid;
+        v[i] = row[min(key, a.kv_len - 1)];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // this wave's 64 keys are one key block
+        const int key = k0 + i * THREADS + tid, blk = (k0 + i * THREADS) / 64 + wave;
+        const uint64_t word = __ballot(key < a.kv_len && v[i] != 0);
+        if (lane == 0 && blk < KEEP_BLOCKS) {
+          skeep[2 * blk] = (uint32_t)word;
+          skeep[2 * blk + 1] = (uint32_t)(word >> 32);
+        }
+        if (word) {
+          lo = min(lo, blk * 64 + __builtin_ctzll(word));
+          hi = max(hi, blk * 64 + 63 - __builtin_clzll(word));
+        }
+      }
+    }
+    int *ends = (int *)&sml[0][0][0];
+    if (lane == 0) {
+      ends[2 * wave] = lo;
+      ends[2 * wave + 1] = hi;
+    }
+    __syncthreads();
+    seen_lo = min(min(ends[0], ends[2]), min(ends[4], ends[6]));
+    seen_hi = max(max(ends[1], ends[3]), max(ends[5], ends[7]));
+    seen_lo = __builtin_amdgcn_readfirstlane(seen_lo);
+    seen_hi = __builtin_amdgcn_readfirstlane(seen_hi);
+    __syncthreads();
+  }
+
   // ---- phases: late query block then early one (causal balance)
-  const int qb_a = a.n_qblocks - 1 - pair, qb_b = pair;
+  const int qb_a = a.n_qblocks - 1 - pair, qb_b = a.single ? qb_a : pair;
   // key blocks [lo, lo + n) that meet a query block's visible key range
   auto key_range = [&](int qb, int &lo, int &n) __attribute__((always_inline)) {
-    int klo = 0, khi = a.kv_len - 1;
+    int klo = seen_lo, khi = seen_hi;
     if (a.flags & F_CAUSAL) khi = min(khi, qb * QB + QB - 1 + a.diag);
-    if (MASK == MASK_GENERAL && (a.flags & F_WINDOW)) klo = max(0, qb * QB + a.lo_off);
+    if (MASK != MASK_CAUSAL && (a.flags & F_WINDOW)) klo = max(klo, qb * QB + a.lo_off);
     if (khi < klo) { lo = 0; n = 0; return; }
     lo = klo / BK;
     n = khi / BK - lo + 1;
@@ -293,23 +361,102 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
     l_part = 0.0f;
   };
 
+  // Mask operands of one block, loaded an iteration before their use (the
+  // loads land behind that iteration's matrix work and its barrier's wait):
+  // keep bytes and bias values of keys 8 r4 + 4 g + 0 .. 3 of key tile kt.
+  uint32_t keep_w[2][4];
+  f32x4 bias_w[MASK == MASK_GENERAL ? 2 : 1][4];
+  auto load_mask = [&](int kb) __attribute__((always_inline)) {
+    if constexpr (MASK != MASK_CAUSAL) {
+      const int qc = min(q0 + l32, a.q_len - 1);
+      if (a.keep && !row_mask) {
+        const uint8_t *krow = a.keep + b * a.keep_sb + h * a.keep_sh + qc * a.keep_sq;
+        if (a.kv_len >= 4) {
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) keep_w[kt][r4] = keep_word(krow, kb * BK + kt * 32 + 8 * r4 + 4 * g, a.kv_len);
+        } else {  // up to three keys
+          uint32_t w = 0;
+          for (int i = 0; i < a.kv_len; ++i) w |= (uint32_t)krow[i] << (8 * i);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) keep_w[q / 4][q % 4] = q == 0 ? w : 0;
+        }
+      }
+      if constexpr (MASK == MASK_GENERAL) {
+        if (a.bias) {
+          const float *brow = a.bias + b * a.bias_sb + h * a.bias_sh + qc * a.bias_sq;
+          const bool whole = kb * BK + BK <= a.kv_len;
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              const int key = kb * BK + kt * 32 + 8 * r4 + 4 * g;
+              if (whole) {
+                __builtin_memcpy(&bias_w[kt][r4], brow + key, 16);
+              } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) bias_w[kt][r4][i] = brow[min(key + i, a.kv_len - 1)];
+              }
+            }
+        } else {
+#pragma unroll
+          for (int q = 0; q < 8; ++q) bias_w[q / 4][q % 4] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      }
+    }
+  };
   // scores of block kb -> the operand of the exponentials (MASK_GENERAL
-  // rewrites S into u = t * log2(e) and uses c_eff = 1)
+  // rewrites S into u = t * log2(e) and uses c_eff = 1; the others keep the
+  // raw score and set -inf where the key is invisible)
   auto mask_scores = [&](int kb, f32x16 (&s)[2]) __attribute__((always_inline)) {
     const int qi = q0 + l32;
-    if constexpr (MASK == MASK_GENERAL) {
-      const int qc = min(qi, a.q_len - 1);
-      const float *brow = a.bias ? a.bias + b * a.bias_sb + h * a.bias_sh + qc * a.bias_sq : nullptr;
-      const uint8_t *krow = a.keep ? a.keep + b * a.keep_sb + h * a.keep_sh + qc * a.keep_sq : nullptr;
+    if constexpr (MASK != MASK_CAUSAL) {
       const int hi_k = (a.flags & F_CAUSAL) ? min(qi + a.diag, a.kv_len - 1) : a.kv_len - 1;
       const int lo_k = (a.flags & F_WINDOW) ? qi + a.lo_off : 0;
+      auto lane_bits = [&](uint32_t w) __attribute__((always_inline)) {
+        const uint32_t x = (w >> (4 * g)) & 0x0f0f0f0fu, y = (x | (x >> 4)) & 0x00ff00ffu;
+        return (y | (y >> 8)) & 0xffffu;
+      };
+      // bit 16 kt + r of `vis`: score r of key tile kt is visible
+      uint32_t vis = 0xffffffffu;
+      const bool inside = kb * BK >= lo_k && kb * BK + BK - 1 <= hi_k;
+      if (!__all(inside)) {
+        // keys of the block up to hi_k and from lo_k, as 64 bits, then this
+        // lane's (bits 8 r4 + 4 g + i of each half, moved to bits 4 r4 + i)
+        const int up = min(max(hi_k - kb * BK + 1, 0), 64), dn = min(max(lo_k - kb * BK, 0), 64);
+        const uint64_t span = (up == 64 ? ~0ull : (1ull << up) - 1) & ~(dn == 64 ? ~0ull : (1ull << dn) - 1);
+        vis = lane_bits((uint32_t)span) | lane_bits((uint32_t)(span >> 32)) << 16;
+      }
+      if (row_mask) {
+        vis &= lane_bits(skeep[2 * kb]) | lane_bits(skeep[2 * kb + 1]) << 16;
+      } else if (a.keep) {
+        uint32_t seen = 0;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb * BK + kt * 32 + 8 * (r >> 2) + 4 * g + (r & 3);
-          s[kt][r] = general_score<T>(s[kt][r], a.scale, a.flags, brow, krow, key, key <= hi_k && key >= lo_k);
-        }
+          for (int r4 = 0; r4 < 4; ++r4) {
+            // bit 7 of every nonzero byte, then the four bits side by side
+            const uint32_t w = keep_w[kt][r4];
+            const uint32_t nz = ((((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) >> 7) & 0x01010101u;
+            seen |= ((nz * 0x10204080u) >> 28) << (16 * kt + 4 * r4);
+          }
+        vis &= seen;
+      }
+      if constexpr (MASK == MASK_GENERAL) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            s[kt][r] = general_score<T>(s[kt][r], a.scale, (a.flags & F_ROUND_SCALED) != 0,
+                                        (a.flags & F_ROUND_BIASED) != 0, bias_w[kt][r >> 2][r & 3],
+                                        (vis & (1u << (16 * kt + r))) != 0);
+      } else if (__any(vis != 0xffffffffu)) {
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[kt][r] = (vis & (1u << (16 * kt + r))) ? s[kt][r] : -__builtin_inff();
+      }
     } else {
       const bool need = ((a.flags & F_CAUSAL) && kb * BK + BK - 1 > q0 + a.diag) || kb * BK + BK > a.kv_len;
       if (need) {
@@ -318,7 +465,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            if (kb * BK + kt * 32 + 8 * (r >> 2) + 4 * g + (r & 3) > lim) s[kt][r] = -__builtin_inff();
+            s[kt][r] = kb * BK + kt * 32 + 8 * (r >> 2) + 4 * g + (r & 3) > lim ? -__builtin_inff() : s[kt][r];
       }
     }
   };
@@ -531,6 +678,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
         for (int r = 0; r < 16; ++r) s_cur[kt][r] = -__builtin_inff();
     } else {
       mask_scores(lo + 2 * u + half, s_cur);
+      if (u + 1 < nh) load_mask(lo + 2 * (u + 1) + half);
     }
     const float rs = body(T1{}, std::integral_constant<bool, !FIRST>{}, T1{}, T1{}, (P ? sk0 : sk1) + half * BLK,
                           (P ? sv0 : sv1) + half * BLK, (P ? sk1 : sk0) + half * BLK + tile * 32 * ROWB,
@@ -546,6 +694,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(1, 1)))
   auto run_phase = [&](int qb, int lo, int tn, int nh, int &t) __attribute__((always_inline)) {
     load_q(qb);
     reset();
+    if (nh > 0) load_mask(lo + half);
     if (tn > 0) {
       {  // prologue: S_0 = QK(0) (K(t) moved two iterations ago)
         const char *kb = kslot(t & 1);
@@ -759,15 +908,34 @@ int attention_prefill_masked(wafer_hip_context *ctx, uint32_t format, const void
   args.keep_sb = m.keep_strides[0];
   args.keep_sh = m.keep_strides[1];
   args.keep_sq = m.keep_strides[2];
-  const bool general = m.bias || m.keep || (m.flags & (WAFER_HIP_ATT_WINDOW | WAFER_HIP_ATT_ROUND_SCALED));
+  // the score region (bias, rounding), else masks alone, else the causal bound alone
+  const bool general = m.bias || (m.flags & WAFER_HIP_ATT_ROUND_SCALED);
+  const bool select = m.keep || (m.flags & WAFER_HIP_ATT_WINDOW);
   WAFER_TRY(check_hip(hipSetDevice(ctx->device), "hipSetDevice"));
   const bool bf = format == WAFER_FMT_BF16;
   if (head_dim == 128 || head_dim == 64) {
-    const dim3 grid((unsigned)(args.bh_count * ((args.n_qblocks + 1) / 2)));
+    // A late and an early query block per workgroup balance the causal walk;
+    // one block each is the finer grain.  With two workgroups per CU (head_dim
+    // 64) the finer grain was never slower (us, pairs / single blocks: causal
+    // 16 heads x 2048 24.7 / 20.0, 4 x 8 x 1500 29.5 / 22.4, full 16 x 2048
+    // 34.2 / 28.1, 8 x 300 13.8 / 7.2).  With one, single blocks serve where
+    // the pairs leave a last round nearly empty or CUs idle; costs in key
+    // blocks, two more per query block for its start and merge.
+    const long n = args.n_qblocks, nk = (kv_len + BK - 1) / BK, cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+    const bool tri = (m.flags & WAFER_HIP_ATT_CAUSAL) != 0;
+    const long pairs = (long)args.bh_count * ((n + 1) / 2), singles = (long)args.bh_count * n;
+    const long cost_pair = ((pairs + cus - 1) / cus) * (tri ? nk + 5 : 2 * nk + 4);
+    const long cost_single = tri ? std::max(nk + 2, (singles * (nk / 2 + 3) + cus - 1) / cus + nk / 4)
+                                 : ((singles + cus - 1) / cus) * (nk + 2);
+    const bool two = fa_waves((int)head_dim, general ? MASK_GENERAL : select ? MASK_SELECT : MASK_CAUSAL) == 2;
+    args.single = singles <= 0x7fffffffL && (two || cost_single < cost_pair);
+    const dim3 grid((unsigned)(args.single ? singles : pairs));
 #define FA_LAUNCH(TT, DD)                                                                              \
   do {                                                                                                 \
     if (general)                                                                                       \
       hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_GENERAL>), grid, dim3(THREADS), 0, ctx->stream, args);   \
+    else if (select)                                                                                   \
+      hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_SELECT>), grid, dim3(THREADS), 0, ctx->stream, args);    \
     else                                                                                               \
       hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_CAUSAL>), grid, dim3(THREADS), 0, ctx->stream, args);    \
   } while (0)
