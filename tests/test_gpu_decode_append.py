@@ -190,3 +190,39 @@ def test_decode_append_rejects_overflow_without_writing(hip):
         hip.attention_decode_append(q, kn, kn, kc, vc, o, 0.1, 3)
     assert L.wafer_hip_attention_decode_append(hip._bind(), BF16, B._p(q), B._p(kn), B._p(kn), B._p(kc), B._p(vc),
                                                B._p(o), 1, 1, 1, 2, 1, 4, 96, 0.1, 16) == -3
+
+
+@pytest.mark.parametrize("fmt", [2, 3], ids=["f16", "bf16"])
+@pytest.mark.parametrize("Bn,Hq,Hkv,L,chunks", [
+    (1, 8, 8, 1, 16), (1, 8, 4, 17, 1), (1, 4, 4, 129, 1), (1, 4, 1, 3231, 16), (2, 8, 1, 1000, 3), (1, 2, 2, 8191, 4),
+    (24, 16, 8, 260, 16), (24, 32, 8, 130, 16), (3, 8, 8, 700, 20)])
+def test_split_chunks_and_fused_append(hip, fmt, Bn, Hq, Hkv, L, chunks):
+    """The chunk grid with chunks split over workgroups (one part of 16 keys to
+    several, parts past the end empty) and the one-workgroup path, against
+    float64 attention under the attention policy; the append step equals the
+    plain decode on the appended cache bit for bit, as does the no-allocation
+    entry, and changes only its own row of the caches."""
+    print("[split decode]", fmt, Bn, Hq, Hkv, L, chunks, flush=True)
+    dt = torch.float16 if fmt == 2 else torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(L + Hq)
+    cap = L + 3
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dt)  # noqa: E731
+    q, k, v, kn, vn = r(Bn, Hq, 1, 128), r(Bn, Hkv, cap, 128), r(Bn, Hkv, cap, 128), r(Bn, Hkv, 1, 128), r(Bn, Hkv, 1, 128)
+    k[:, :, L:] = float("nan")
+    v[:, :, L:] = float("nan")
+    kc, vc = k.clone(), v.clone()
+    k[:, :, L - 1:L], v[:, :, L - 1:L] = kn, vn
+    o, oa, on = (torch.zeros_like(q) for _ in range(3))
+    scale = 128 ** -0.5
+    hip.attention_decode(q, k, v, o, scale, chunks=chunks, kv_len=L, fmt=fmt)
+    hip.attention_decode_append(q, kn, vn, kc, vc, oa, scale, L - 1, chunks=chunks, fmt=fmt)
+    if Bn * Hq * chunks <= 8192:  # what the no-allocation scratch holds
+        hip.attention_decode_noalloc(q, k, v, on, scale, chunks=chunks, kv_len=L, fmt=fmt)
+    else:
+        on = o
+    bits = lambda t: t.view(torch.int16)  # noqa: E731
+    assert torch.equal(bits(o), bits(oa)) and torch.equal(bits(o), bits(on))
+    assert torch.equal(bits(kc), bits(k)) and torch.equal(bits(vc), bits(v))
+    kk, vv = (t[:, :, :L].double().cpu().repeat_interleave(Hq // Hkv, dim=1) for t in (k, v))
+    p = torch.softmax(q.double().cpu() @ kk.transpose(2, 3).contiguous() * scale, dim=-1)
+    attention_gate(o.float().cpu().numpy(), (p @ vv).float().numpy(), what="split decode")

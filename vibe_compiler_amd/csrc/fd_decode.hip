@@ -28,7 +28,12 @@
 //    folded left to right through LDS, so there is a single launch and no
 //    cross-workgroup traffic;
 //  * small batches: a grid of (chunk, kv_head, batch) workgroups writes chunk
-//    states to the context workspace and a second launch folds them.
+//    states to the context workspace and a second launch folds them; where
+//    that grid leaves CUs idle each chunk is split over 2 .. workgroups (32
+//    heads over 8 KV heads, one sequence of 8192 keys: 20.4 -> 13.5 us; 8 over
+//    4, 3231 keys: 13.2 -> 9.2 us);
+//  * a decode step's new K / V row is read from the step's tensors and written
+//    to the cache by the wave that owns it, without a launch of its own.
 // Scores are tracked in the log2 domain (m2 = m * scale * log2e) so every
 // ExpLp becomes one exp2 of an fma; see fa_prefill.hip for the rounding note.
 #include "common.h"
@@ -88,14 +93,16 @@ __device__ inline void wave_lds_order() {
 // Online state of one wave over keys [k0, k1), for the G query heads of a
 // GQA group.  On return, lanes with grp == 0 hold acc[h][hl*8 + e]; every
 // lane holds m2 / l of head (lane & 15) (meaningful for heads < G).
-template <typename T, int G>
+// APPEND: row `past` of the cache is the step's new row, read from kn / vn
+// (the wave that owns it also writes it to the cache: append_row).
+template <typename T, int G, bool APPEND>
 struct WaveSweep {
   float m2, lsum;
   float acc[G][8];
 
   __device__ void run(const uint16_t *__restrict__ Kp, const uint16_t *__restrict__ Vp,
                       const v8<T> (&qreg)[4], int k0, int k1, int nblk, float c,
-                      float (*sP)[G]) {
+                      float (*sP)[G], const uint16_t *__restrict__ kn, const uint16_t *__restrict__ vn, int past) {
     const int lane = threadIdx.x & 63, hl = lane & 15, grp = lane >> 4;
     m2 = -__builtin_inff();
     lsum = 0.0f;
@@ -114,7 +121,9 @@ struct WaveSweep {
       for (int gi = 0; gi < 2; ++gi) {
         const int key = kbase + gi * 16 + hl;
         const bool ok = key < k1;
-        const uint16_t *kr = Kp + (size_t)(ok ? key : 0) * D + grp * 8;
+        const uint16_t *row = Kp + (size_t)(ok ? key : 0) * D;
+        if (APPEND) row = key == past ? kn : row;
+        const uint16_t *kr = row + grp * 8;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           kreg[gi][s] = __builtin_nontemporal_load((const v8<T> *)(kr + s * 32));
@@ -128,7 +137,9 @@ struct WaveSweep {
       for (int i = 0; i < BLK / 4; ++i) {
         const int key = kbase + grp + 4 * i;
         const bool ok = key < k1;
-        vreg[i] = __builtin_nontemporal_load((const u32x4 *)(Vp + (size_t)(ok ? key : 0) * D + hl * 8));
+        const uint16_t *row = Vp + (size_t)(ok ? key : 0) * D;
+        if (APPEND) row = key == past ? vn : row;
+        vreg[i] = __builtin_nontemporal_load((const u32x4 *)(row + hl * 8));
         if (!ok) vreg[i] = u32x4{0u, 0u, 0u, 0u};
       }
       // S^T = K . Q^T : lane holds head hl, keys gi*16 + 4 grp + r
@@ -202,6 +213,16 @@ struct WaveSweep {
   }
 };
 
+// The new K and V rows of one (batch, kv head), 16 bytes per lane, byte for
+// byte, into row `past` of its caches.
+__device__ inline void append_row(uint16_t *kp, uint16_t *vp, const uint16_t *kn, const uint16_t *vn, int past) {
+  const int lane = threadIdx.x & 63, hl = lane & 15;
+  if (lane < 32) {
+    uint16_t *dst = (lane < 16 ? kp : vp) + (size_t)past * D + hl * 8;
+    *(u32x4 *)dst = *(const u32x4 *)((lane < 16 ? kn : vn) + hl * 8);
+  }
+}
+
 __device__ inline void merge(float &m, float &l, float &a, float mr, float lr, float ar) {
   const float mm = fmaxf(m, mr);
   const float e = (mm == -__builtin_inff()) ? 0.0f : mm;
@@ -224,8 +245,8 @@ __device__ inline void load_q(const uint16_t *__restrict__ Q, int row_base, int 
   }
 }
 
-template <typename T, int G>
-__device__ inline void publish_state(const WaveSweep<T, G> &st, int wave, float (*sAcc)[G][D],
+template <typename T, int G, bool APPEND>
+__device__ inline void publish_state(const WaveSweep<T, G, APPEND> &st, int wave, float (*sAcc)[G][D],
                                      float (*sM)[G], float (*sL)[G]) {
   const int lane = threadIdx.x & 63, hl = lane & 15, grp = lane >> 4;
   if (grp == 0) {
@@ -243,11 +264,12 @@ __device__ inline void publish_state(const WaveSweep<T, G> &st, int wave, float 
 // ---- one workgroup (16 waves) per (batch, kv_head) ----------------------------
 constexpr int WG_WAVES = 16;
 
-template <typename T, int G>
+template <typename T, int G, bool APPEND>
 __global__ __launch_bounds__(1024) void fd_group_d128(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ Kc,
     const uint16_t *__restrict__ Vc, uint16_t *__restrict__ O, int q_heads, int kv_heads,
-    int kv_len, int cap, int chunks, int chunk_len, int sub, float c) {
+    int kv_len, int cap, int chunks, int chunk_len, int sub, float c, const uint16_t *__restrict__ Kn,
+    const uint16_t *__restrict__ Vn) {
   __shared__ float sP[WG_WAVES][BLK][G];
   __shared__ float sAcc[WG_WAVES][G][D];
   __shared__ float sM[WG_WAVES][G], sL[WG_WAVES][G];
@@ -268,9 +290,12 @@ __global__ __launch_bounds__(1024) void fd_group_d128(
 
   v8<T> qreg[4];
   load_q<T>(Q, row_base, G, qreg);
-  WaveSweep<T, G> st;
-  st.run(Kp, Vp, qreg, k0, k1, (k1 - k0 + BLK - 1) / BLK, c, sP[wave]);
-  publish_state<T, G>(st, wave, sAcc, sM, sL);
+  WaveSweep<T, G, APPEND> st;
+  const size_t new_row = (size_t)(b * kv_heads + kvh) * D;
+  st.run(Kp, Vp, qreg, k0, k1, (k1 - k0 + BLK - 1) / BLK, c, sP[wave], Kn + new_row, Vn + new_row, kv_len - 1);
+  if (APPEND && k0 <= kv_len - 1 && kv_len - 1 < k1)
+    append_row((uint16_t *)Kp, (uint16_t *)Vp, Kn + new_row, Vn + new_row, kv_len - 1);
+  publish_state<T, G, APPEND>(st, wave, sAcc, sM, sL);
   __syncthreads();
   // left fold over the wave states in key order (= chunk order), finalize
   const int used = min(WG_WAVES, chunks * sub);
@@ -284,11 +309,14 @@ __global__ __launch_bounds__(1024) void fd_group_d128(
 }
 
 // ---- chunk grid + separate fold (small batches) --------------------------------
-template <typename T, int G>
+// A chunk may be split over `sub` workgroups (parts of sub_len keys), whose
+// states fold left to right like chunks of their own: `states` = chunks * sub.
+template <typename T, int G, bool APPEND>
 __global__ __launch_bounds__(256) void fd_chunk_d128(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ Kc,
     const uint16_t *__restrict__ Vc, ChunkState *__restrict__ part, int q_heads, int kv_heads,
-    int kv_len, int cap, int chunk_len, int chunks, float c) {
+    int kv_len, int cap, int chunk_len, int states, int sub, int sub_len, float c, const uint16_t *__restrict__ Kn,
+    const uint16_t *__restrict__ Vn) {
   __shared__ float sP[4][BLK][G];
   __shared__ float sAcc[4][G][D];
   __shared__ float sM[4][G], sL[4][G];
@@ -299,8 +327,10 @@ __global__ __launch_bounds__(256) void fd_chunk_d128(
   const uint16_t *Vp = Vc + ((size_t)(b * kv_heads + kvh) * cap) * D;
   const int row_base = b * q_heads + kvh * G;
 
-  const int c0 = ch * chunk_len;
-  const int c1 = min(c0 + chunk_len, kv_len);
+  const int chunk = ch / sub, piece = ch - chunk * sub;
+  const int cend = min(chunk * chunk_len + chunk_len, kv_len);
+  const int c0 = chunk * chunk_len + piece * sub_len;
+  const int c1 = min(c0 + sub_len, cend);
   const int n = max(c1 - c0, 0);
   const int per = ((n + 4 * 16 - 1) / (4 * 16)) * 16;
   int k0 = c0 + wave * per;
@@ -309,16 +339,19 @@ __global__ __launch_bounds__(256) void fd_chunk_d128(
 
   v8<T> qreg[4];
   load_q<T>(Q, row_base, G, qreg);
-  WaveSweep<T, G> st;
-  st.run(Kp, Vp, qreg, k0, k1, (k1 - k0 + BLK - 1) / BLK, c, sP[wave]);
-  publish_state<T, G>(st, wave, sAcc, sM, sL);
+  WaveSweep<T, G, APPEND> st;
+  const size_t new_row = (size_t)(b * kv_heads + kvh) * D;
+  st.run(Kp, Vp, qreg, k0, k1, (k1 - k0 + BLK - 1) / BLK, c, sP[wave], Kn + new_row, Vn + new_row, kv_len - 1);
+  if (APPEND && k0 <= kv_len - 1 && kv_len - 1 < k1)
+    append_row((uint16_t *)Kp, (uint16_t *)Vp, Kn + new_row, Vn + new_row, kv_len - 1);
+  publish_state<T, G, APPEND>(st, wave, sAcc, sM, sL);
   __syncthreads();
   for (int idx = threadIdx.x; idx < G * D; idx += 256) {
     const int h = idx / D, d = idx % D;
     float m = sM[0][h], l = sL[0][h], a = sAcc[0][h][d];
 #pragma unroll
     for (int w = 1; w < 4; ++w) merge(m, l, a, sM[w][h], sL[w][h], sAcc[w][h][d]);
-    ChunkState &cs = part[(size_t)(row_base + h) * chunks + ch];
+    ChunkState &cs = part[(size_t)(row_base + h) * states + ch];
     cs.acc[d] = a;
     if (d == 0) {
       cs.m2 = m;
@@ -328,13 +361,50 @@ __global__ __launch_bounds__(256) void fd_chunk_d128(
 }
 
 // Left fold over the chunk states of one (batch, q_head), then finalize.
-template <typename T>
-__global__ __launch_bounds__(128) void fd_fold_d128(const ChunkState *__restrict__ part, uint16_t *__restrict__ O,
-                                                    int chunks) {
-  const int bh = blockIdx.x, d = threadIdx.x;
-  const ChunkState *ps = part + (size_t)bh * chunks;
-  float m = ps[0].m2, l = ps[0].l, a = ps[0].acc[d];
-  for (int cc = 1; cc < chunks; ++cc) merge(m, l, a, ps[cc].m2, ps[cc].l, ps[cc].acc[d]);
+// What bounds it is latency: one thread per d folding every state took 5.9 us
+// for 16 states.  P groups of 128 threads each fold a run of the states, the
+// loads of 8 states out together, and the runs' states fold left to right
+// through LDS.  A decode step over 32 x 4095 keys (append, chunks, fold):
+// 20.7 -> 15.7 us.
+template <typename T, int P>
+__global__ __launch_bounds__(128 * P) void fd_fold_d128(const ChunkState *__restrict__ part,
+                                                        uint16_t *__restrict__ O, int states) {
+  constexpr int NB = 8;
+  __shared__ float sA[P][D], sM[P], sL[P];
+  const int bh = blockIdx.x, d = threadIdx.x % D, run = threadIdx.x / D;
+  const ChunkState *ps = part + (size_t)bh * states;
+  const int per = (states + P - 1) / P, s0 = run * per, s1 = min(s0 + per, states);
+  float m = -__builtin_inff(), l = 0.0f, a = 0.0f;
+  for (int c0 = s0; c0 < s1; c0 += NB) {
+    float mr[NB], lr[NB], ar[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      const ChunkState &cs = ps[min(c0 + i, s1 - 1)];
+      mr[i] = cs.m2;
+      lr[i] = cs.l;
+      ar[i] = cs.acc[d];
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      if (c0 + i == s0) {
+        m = mr[i];
+        l = lr[i];
+        a = ar[i];
+      } else if (c0 + i < s1) {
+        merge(m, l, a, mr[i], lr[i], ar[i]);
+      }
+    }
+  }
+  sA[run][d] = a;
+  if (d == 0) {
+    sM[run] = m;
+    sL[run] = l;
+  }
+  __syncthreads();
+  if (run != 0) return;
+#pragma unroll
+  for (int r = 1; r < P; ++r)
+    if (r * per < states) merge(m, l, a, sM[r], sL[r], sA[r][d]);
   const float coef = (l == 0.0f) ? 0.0f : 1.0f / l;
   O[(size_t)bh * D + d] = narrow<T>(a * coef);
 }
@@ -363,12 +433,24 @@ int scratch_for(int device, ChunkState **out) {
   return WAFER_HIP_OK;
 }
 
-// Shared by both entries: validation, then the group path (no workspace) or
-// the chunk grid plus fold, whose states go to `part` when given, else to
-// the context's workspace (grown on demand).
+// Whether a call runs one workgroup per (batch, kv head).  (G = 8 needs more
+// than the 128 VGPRs of a 16-wave workgroup, and so does the F16 kernel for
+// G = 4: those take the chunk grid.)
+bool takes_group(const wafer_hip_context *ctx, uint32_t format, uint32_t G, uint32_t chunks, uint32_t batch,
+                 uint32_t kv_heads) {
+  const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const uint32_t gmax = format == WAFER_FMT_BF16 ? 4u : 2u;
+  return G <= gmax && chunks <= (uint32_t)WG_WAVES && (uint64_t)batch * kv_heads * 4 >= (uint64_t)cus * 3;
+}
+
+// Shared by the entries: validation, then the group path (no workspace) or
+// the chunk grid plus fold, whose states go to the no-allocation scratch or to
+// the context's workspace (grown on demand).  k_new / v_new: row kv_len - 1 of
+// the caches is the step's new row, taken from there and written to the caches.
 int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k_cache, const void *v_cache, void *o,
            uint32_t batch, uint32_t q_heads, uint32_t kv_heads, uint32_t kv_len, uint32_t kv_capacity,
-           uint32_t head_dim, float scale, uint32_t chunks, bool noalloc) {
+           uint32_t head_dim, float scale, uint32_t chunks, bool noalloc, const void *k_new = nullptr,
+           const void *v_new = nullptr) {
   WAFER_CHECK_CTX(ctx);
   if (format != WAFER_FMT_BF16 && format != WAFER_FMT_F16)
     return fail(WAFER_HIP_E_UNSUPPORTED, "attention_decode: storage must be BF16 or F16");
@@ -392,10 +474,7 @@ int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k
   // state and is served as well.
   const int chunk_len = (int)((kv_len + chunks - 1) / chunks);
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  // (the F16 group kernel for G = 4 would spill at the 128 VGPRs of a
-  // 16-wave workgroup: F16 groups of 4 take the chunk grid)
-  const uint32_t gmax = format == WAFER_FMT_BF16 ? 4u : 2u;
-  const bool group = G <= gmax && chunks <= (uint32_t)WG_WAVES && (uint64_t)batch * kv_heads * 4 >= (uint64_t)cus * 3;
+  const bool group = takes_group(ctx, format, G, chunks, batch, kv_heads);
   const size_t states = (size_t)batch * q_heads * chunks;
   if (noalloc && !group && states > SCRATCH_STATES)
     return fail(WAFER_HIP_E_UNSUPPORTED, "attention_decode_noalloc: batch * q_heads * chunks = " +
@@ -404,20 +483,24 @@ int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k
   WAFER_TRY(check_hip(hipSetDevice(ctx->device), "hipSetDevice"));
   const float c = scale * 0x1.715476p+0f;
 
-  // (G = 8 needs more than the 128 VGPRs a 16-wave workgroup allows)
   if (group) {
     const int sub = WG_WAVES / (int)chunks;
     dim3 grid(kv_heads, batch);
-#define FD_GROUP(TT, GV)                                                                          \
-  hipLaunchKernelGGL((fd_group_d128<TT, GV>), grid, dim3(1024), 0, ctx->stream, (const uint16_t *)q, \
+#define FD_GROUP1(TT, GV, AP)                                                                     \
+  hipLaunchKernelGGL((fd_group_d128<TT, GV, AP>), grid, dim3(1024), 0, ctx->stream, (const uint16_t *)q, \
                      (const uint16_t *)k_cache, (const uint16_t *)v_cache, (uint16_t *)o,        \
                      (int)q_heads, (int)kv_heads, (int)kv_len, (int)kv_capacity, (int)chunks,    \
-                     chunk_len, sub, c)
+                     chunk_len, sub, c, (const uint16_t *)k_new, (const uint16_t *)v_new)
+#define FD_GROUP(TT, GV)                 \
+  do {                                   \
+    if (k_new) FD_GROUP1(TT, GV, true);  \
+    else FD_GROUP1(TT, GV, false);       \
+  } while (0)
     if (format == WAFER_FMT_BF16) {
       switch (G) {
       case 1: FD_GROUP(__bf16, 1); break;
       case 2: FD_GROUP(__bf16, 2); break;
-      default: FD_GROUP(__bf16, 4); break;
+      default: FD_GROUP1(__bf16, 4, false); break;  // (with the append it would spill)
       }
     } else {
       switch (G) {
@@ -426,21 +509,40 @@ int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k
       }
     }
 #undef FD_GROUP
+#undef FD_GROUP1
     return launch_status("fd_group_d128");
   }
 
+  // Chunks split over workgroups until there are two for every CU, in parts
+  // of 128 keys at least (one 32-key step per wave), and never past the states
+  // the no-allocation scratch holds, so both entries split alike.
+  int sub = 1;
+  while ((uint64_t)chunks * sub * kv_heads * batch < 2 * (uint64_t)cus && chunk_len > 128 * sub &&
+         states * 2 * sub <= SCRATCH_STATES)
+    sub *= 2;
+  const int sub_len = (((chunk_len + sub - 1) / sub) + 15) / 16 * 16;
+  const int nstates = (int)chunks * sub;
   ChunkState *part = nullptr;
   if (noalloc) {
     WAFER_TRY(scratch_for(ctx->device, &part));
   } else {
-    WAFER_TRY(ensure_workspace(ctx, &ctx->workspace, &ctx->workspace_bytes, states * sizeof(ChunkState)));
+    // at least what any split grid needs, so that a call sized by one shape
+    // serves the other split shapes too
+    WAFER_TRY(ensure_workspace(ctx, &ctx->workspace, &ctx->workspace_bytes,
+                               std::max(states * sub, SCRATCH_STATES) * sizeof(ChunkState)));
     part = (ChunkState *)ctx->workspace;
   }
-  dim3 grid(chunks, kv_heads, batch);
-#define FD_CHUNK(TT, GV)                                                                          \
-  hipLaunchKernelGGL((fd_chunk_d128<TT, GV>), grid, dim3(256), 0, ctx->stream, (const uint16_t *)q, \
+  dim3 grid((unsigned)nstates, kv_heads, batch);
+#define FD_CHUNK1(TT, GV, AP)                                                                     \
+  hipLaunchKernelGGL((fd_chunk_d128<TT, GV, AP>), grid, dim3(256), 0, ctx->stream, (const uint16_t *)q, \
                      (const uint16_t *)k_cache, (const uint16_t *)v_cache, part, (int)q_heads,    \
-                     (int)kv_heads, (int)kv_len, (int)kv_capacity, chunk_len, (int)chunks, c)
+                     (int)kv_heads, (int)kv_len, (int)kv_capacity, chunk_len, nstates, sub, sub_len, c, \
+                     (const uint16_t *)k_new, (const uint16_t *)v_new)
+#define FD_CHUNK(TT, GV)                 \
+  do {                                   \
+    if (k_new) FD_CHUNK1(TT, GV, true);  \
+    else FD_CHUNK1(TT, GV, false);       \
+  } while (0)
   if (format == WAFER_FMT_BF16) {
     switch (G) {
     case 1: FD_CHUNK(__bf16, 1); break;
@@ -457,13 +559,19 @@ int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k
     }
   }
 #undef FD_CHUNK
+#undef FD_CHUNK1
   WAFER_TRY(launch_status("fd_chunk_d128"));
-  if (format == WAFER_FMT_BF16)
-    hipLaunchKernelGGL(fd_fold_d128<__bf16>, dim3(batch * q_heads), dim3(D), 0, ctx->stream, part, (uint16_t *)o,
-                       (int)chunks);
-  else
-    hipLaunchKernelGGL(fd_fold_d128<_Float16>, dim3(batch * q_heads), dim3(D), 0, ctx->stream, part, (uint16_t *)o,
-                       (int)chunks);
+#define FD_FOLD(TT, PV)                                                                                      \
+  hipLaunchKernelGGL((fd_fold_d128<TT, PV>), dim3(batch * q_heads), dim3(D * PV), 0, ctx->stream, part, (uint16_t *)o, \
+                     nstates)
+  if (format == WAFER_FMT_BF16) {
+    if (nstates > 16) FD_FOLD(__bf16, 8);
+    else FD_FOLD(__bf16, 2);
+  } else {
+    if (nstates > 16) FD_FOLD(_Float16, 8);
+    else FD_FOLD(_Float16, 2);
+  }
+#undef FD_FOLD
   return launch_status("fd_fold_d128");
 }
 
@@ -567,6 +675,11 @@ extern "C" int wafer_hip_attention_decode_append(wafer_hip_context *ctx, uint32_
   // the append: whole 16-byte pieces when every row is, else per element
   const bool vec = head_dim % 8 == 0 &&
                    (((uintptr_t)k_new | (uintptr_t)v_new | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
+  // one token at head_dim 128: the decode kernels write the new rows
+  // themselves (a launch of 1.7 us and its gap less)
+  if (fd && vec && !(q_heads / kv_heads == 4 && takes_group(ctx, format, 4, chunks, batch, kv_heads)))
+    return decode(ctx, format, q, k_cache, v_cache, o, batch, q_heads, kv_heads, past_len + 1, kv_capacity, head_dim,
+                  scale, chunks, false, k_new, v_new);
   const int piece_elems = vec ? 8 : 1;
   const int row_pieces = (int)head_dim / piece_elems;
   const int64_t pieces = (int64_t)batch * kv_heads * tokens * row_pieces;
