@@ -23,11 +23,6 @@ enum { KIND_BF16 = 0, KIND_F16 = 1, KIND_I8 = 2 };
 // element is read before it is written, by the same lane).
 enum { OUT_F32 = 0, OUT_NARROW = 1, OUT_I8_DEQUANT = 2, OUT_SWIGLU = 3, OUT_NARROW_RES = 4 };
 
-// f16 -> f32 by v_cvt_f32_f16: exact for every finite f16 (subnormals
-// included, f16 denormals are on); a NaN keeps a NaN, and the sum it enters
-// narrows to the canonical f16 NaN either way, so the residual sum matches
-// the portable widening bit for bit.
-__device__ inline float widen_f16(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 // f32 -> f16 by v_cvt_f16_f32 in the default round-to-nearest-even mode, with
 // gradual underflow and overflow to +-inf; a NaN narrows to the canonical
 // 0x7e00 as f32_to_f16 does.
