@@ -111,3 +111,34 @@ def test_gemm_i8_rows_bit_exact(hip, B, m, n, k, rt):
                 n, rhs_t=rt)  # without the accumulators: the staged stores
     assert torch.equal(y[:m * n].view(m, n).cpu(), yref)
     assert torch.all(acc[m * n:] == 0) and torch.all(y[m * n:] == 0)
+
+
+@pytest.mark.parametrize("m,k,n,batch,fmt,lt", [
+    (1, 40, 57400, 1, 5, 0), (2, 5, 65000, 1, 5, 1), (3, 1000, 1000, 1, 3, 0), (9, 17, 130, 1, 2, 1), (16, 300, 700, 1, 2, 0),
+    (130, 512, 2000, 1, 5, 0), (127, 31, 2001, 1, 5, 1), (300, 80, 1500, 1, 5, 1), (129, 63, 1030, 1, 3, 1),
+    (257, 33, 2047, 1, 2, 0), (65, 15, 64, 120, 5, 0), (5, 48, 100, 300, 3, 1)])
+def test_formal_gemm_rows_bit_exact(hip, B, oracle, m, k, n, batch, fmt, lt):
+    """The formal GEMM's register chains at the edges of their row tiles, 64
+    columns and 16-k chunks (fewer k than one chunk, a partial last one), with
+    zeros of both signs, an infinity and a NaN among the operands, a partial sum
+    and both lhs orientations, bit for bit against the oracle."""
+    print("[formal rows]", m, k, n, batch, fmt, lt, flush=True)
+    rng = np.random.default_rng(m + 3 * k + n)
+    a = rng.standard_normal((batch, m, k)).astype(np.float32)
+    b = rng.standard_normal((batch, k, n)).astype(np.float32)
+    a[:, 0] = -0.0
+    b[:, :, -1] = 0.0
+    b[:, :, 0] = np.inf
+    b[0, k // 2, n // 2] = np.nan
+    psum = rng.standard_normal((batch, m, n)).astype(np.float32)
+    store = {5: lambda x: x, 3: lambda x: oracle.f32_to_bf16(x).reshape(x.shape),
+             2: lambda x: x.astype(np.float16).view(np.uint16)}[fmt]
+    ah, bh = store(a), store(b)
+    al = np.ascontiguousarray(ah.transpose(0, 2, 1)) if lt else ah
+    ref = oracle.gemm_formal(fmt, fmt, al, bh, m, k, n, batch=batch, psum=psum, lhs_t=bool(lt))
+    dev = lambda x: torch.from_numpy(x.view(np.int16) if x.dtype == np.uint16 else x).cuda()  # noqa: E731
+    out = torch.zeros(batch * m * n + 64, dtype=torch.float32 if fmt == 5 else torch.int16, device="cuda")
+    hip.gemm(dev(al), dev(bh), out, m, k, n, batch=batch, in_fmt=fmt, out_fmt=fmt, psum=dev(psum), lhs_t=bool(lt))
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:-64].view(np.uint32 if fmt == 5 else np.uint16), ref.ravel().view(np.uint32 if fmt == 5 else np.uint16))
+    assert not got[-64:].any()

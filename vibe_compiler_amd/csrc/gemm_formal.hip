@@ -19,7 +19,8 @@
 // each operand with one ds_read_b128; the next slice's global loads are
 // issued before the current slice's chains run.  MT is the largest of 4, 2,
 // 1 whose grid still covers the CUs (a chain is sequential in k, so
-// parallelism comes only from outputs).
+// parallelism comes only from outputs).  A normal rhs takes the LDS-free
+// gemm_formal_rows_kernel where its grid fills the SIMDs.
 #include "common.h"
 
 namespace wafer {
@@ -134,6 +135,178 @@ __global__ __launch_bounds__(256) void gemm_formal_kernel(
     }
 }
 
+// Sixteen steps of R chains: acc[r] = fma(lane j of a[r]'s 16-lane row, b[j],
+// acc[r]) for j = 0 .. 15, the broadcast in the fma itself (v_fmac_f32 with a
+// DPP row broadcast; the compiler makes a move and an fma of the builtins).
+// The s_nop covers a VALU write of an operand just before (two wait states
+// before a DPP read).  Every lane takes part.
+#define FMAC(ACC, A, J, B) "v_fmac_f32_dpp %" ACC ", %" A ", %" B " row_newbcast:" J " row_mask:0xf bank_mask:0xf\n\t"
+#define FMAC1(J, B) FMAC("0", "1", J, B)
+#define FMAC4(J, B) FMAC("0", "4", J, B) FMAC("1", "5", J, B) FMAC("2", "6", J, B) FMAC("3", "7", J, B)
+#define CHAIN_B(b)                                                                                               \
+  "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(b[4]), "v"(b[5]), "v"(b[6]), "v"(b[7]), "v"(b[8]), "v"(b[9]), \
+      "v"(b[10]), "v"(b[11]), "v"(b[12]), "v"(b[13]), "v"(b[14]), "v"(b[15])
+__device__ __attribute__((always_inline)) inline void chain16x1(const float *a, const float (&b)[16], float *acc) {
+  asm("s_nop 1\n\t"
+      FMAC1("0", "2") FMAC1("1", "3") FMAC1("2", "4") FMAC1("3", "5") FMAC1("4", "6")
+      FMAC1("5", "7") FMAC1("6", "8") FMAC1("7", "9") FMAC1("8", "10") FMAC1("9", "11")
+      FMAC1("10", "12") FMAC1("11", "13") FMAC1("12", "14") FMAC1("13", "15") FMAC1("14", "16")
+      FMAC1("15", "17")
+      : "+v"(acc[0])
+      : "v"(a[0]), CHAIN_B(b));
+}
+__device__ __attribute__((always_inline)) inline void chain16x4(const float *a, const float (&b)[16], float *acc) {
+  asm("s_nop 1\n\t"
+      FMAC4("0", "8") FMAC4("1", "9") FMAC4("2", "10") FMAC4("3", "11") FMAC4("4", "12")
+      FMAC4("5", "13") FMAC4("6", "14") FMAC4("7", "15") FMAC4("8", "16") FMAC4("9", "17")
+      FMAC4("10", "18") FMAC4("11", "19") FMAC4("12", "20") FMAC4("13", "21") FMAC4("14", "22")
+      FMAC4("15", "23")
+      : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
+      : "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]), CHAIN_B(b));
+}
+#undef CHAIN_B
+#undef FMAC4
+#undef FMAC1
+#undef FMAC
+// the same for any number of steps and rows, a move and an fma per step
+template <int J, int R>
+__device__ __attribute__((always_inline)) inline void chain_step(const float (&a)[R], const float (&b)[16],
+                                                                 float (&acc)[R], int steps) {
+  if constexpr (J < 16) {
+    if (J < steps) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int s = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, a[r]), 0x150 + J, 0xf, 0xf, true);
+        acc[r] = __builtin_fmaf(__builtin_bit_cast(float, s), b[J], acc[r]);
+      }
+      chain_step<J + 1, R>(a, b, acc, steps);
+    }
+  }
+}
+template <int R>
+__device__ __attribute__((always_inline)) inline void chain16(const float (&a)[R], const float (&b)[16],
+                                                              float (&acc)[R]) {
+  if constexpr (R == 1) chain16x1(a, b, acc);
+  else {
+#pragma unroll
+    for (int r = 0; r < R; r += 4) chain16x4(a + r, b, acc + r);
+  }
+}
+
+// Normal rhs [K, N]: a wave owns R rows x 64 columns, one column per lane and
+// R chains per lane.  What bounds the tiled kernel above is the LDS: two
+// operand reads per pair of fma.  Here the lhs of 16 k sits in one register
+// per row (lane j of every 16-lane row holds k0 + j) and reaches the fma by a
+// DPP row broadcast, and the rhs comes straight from global memory, 64
+// consecutive columns of one k per load, three chunks of 16 k ahead, so there
+// is no LDS at all.  The four waves of a workgroup take row tiles of the same
+// columns and share the rhs in L1.  Same chains, same bits; measured (us, tiled
+// -> here): F32 128 x 512 x 2048 17.6 -> 12.0, 256 x 1024 x 2048 39 -> 27.8,
+// 1024 x 512 x 2048 80 -> 48.5; BF16 128 x 512 x 2048 28.5 -> 13.8, 2000 x 300 x
+// 2000 158 -> 59.
+template <uint32_t IN, uint32_t OUT, int R>
+__global__ __launch_bounds__(256) void gemm_formal_rows_kernel(const void *__restrict__ lhs,
+                                                               const void *__restrict__ rhs,
+                                                               void *__restrict__ dst, const float *__restrict__ psum,
+                                                               int m, int k, int n, int lhs_t, int row_tiles) {
+  constexpr int NB = 4;  // chunks of 16 k in registers
+  const int lane = threadIdx.x & 63;
+  const int id = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = (id % row_tiles) * R, n0 = (id / row_tiles) * 64;
+  if (n0 >= n) return;
+  const int b = blockIdx.z;
+  const int64_t lb = (int64_t)b * m * k, rb = (int64_t)b * k * n, ob = (int64_t)b * m * n;
+  const int col = min(n0 + lane, n - 1), kl = lane & 15;
+
+  // Buffer loads: a wave-uniform base that moves with the chunk, a lane
+  // offset and a scalar offset per row (lhs) or k (rhs), all set up once, so
+  // the loop issues little beside its loads and fma.
+  constexpr int ES = IN == WAFER_FMT_F32 ? 4 : 2;
+  const uint32_t a_k = (uint32_t)(lhs_t ? m : 1) * ES, a_row = (uint32_t)(lhs_t ? 1 : k) * ES, b_k = (uint32_t)n * ES;
+  const char *const abase = (const char *)lhs + (lb + (lhs_t ? m0 : (int64_t)m0 * k)) * ES;
+  const char *const bbase = (const char *)rhs + (rb + n0) * ES;
+  const uint32_t a_off = kl * a_k, b_off = (uint32_t)(col - n0) * ES;
+  auto one = [&](__amdgpu_buffer_rsrc_t r, uint32_t vo, uint32_t so) __attribute__((always_inline)) -> float {
+    if constexpr (IN == WAFER_FMT_F32) {
+      return u2f(__builtin_amdgcn_raw_buffer_load_b32(r, vo, so, 0));
+    } else {
+      const uint16_t h = __builtin_amdgcn_raw_buffer_load_b16(r, vo, so, 0);
+      return IN == WAFER_FMT_BF16 ? bf16_to_f32(h) : widen_f16(h);
+    }
+  };
+  float av[NB + 1][R], bv[NB + 1][16], acc[R];  // the last set: the partial chunk
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+  // `steps` k from 16 c on (16, or what is left: the last k again past it)
+  auto load = [&](int c, int s, int steps) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t ra =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(abase + (int64_t)c * 16 * a_k), 0, -1, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rbv =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(bbase + (int64_t)c * 16 * b_k), 0, -1, 0x00020000);
+    const uint32_t ao = steps == 16 ? a_off : min(kl, steps - 1) * a_k;
+#pragma unroll
+    for (int r = 0; r < R; ++r) av[s][r] = one(ra, ao, (uint32_t)min(r, m - 1 - m0) * a_row);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) bv[s][j] = one(rbv, b_off, (uint32_t)(steps == 16 ? j : min(j, steps - 1)) * b_k);
+  };
+  const int whole = k / 16;
+  if (k % 16 != 0) load(whole, NB, k % 16);
+  if (whole > 0) {
+    const int last = whole - 1;  // loads past it take it again, never used
+#pragma unroll
+    for (int s = 0; s < NB - 1; ++s) load(min(s, last), s, 16);
+    int c = 0;
+    for (; c + NB <= whole; c += NB) {
+#pragma unroll
+      for (int s = 0; s < NB; ++s) {
+        load(min(c + s + NB - 1, last), (s + NB - 1) % NB, 16);
+        __builtin_amdgcn_sched_barrier(0);
+        chain16<R>(av[s], bv[s], acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < NB - 1; ++s)
+      if (c + s < whole) chain16<R>(av[s], bv[s], acc);
+  }
+  // the last k, exactly as many steps as there are (a padded fma(0, 0, -0)
+  // would turn a -0 accumulator into +0)
+  if (k % 16 != 0) chain_step<0, R>(av[NB], bv[NB], acc, k % 16);
+  if (n0 + lane >= n) return;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (m0 + r >= m) continue;
+    float v = acc[r];
+    const int64_t o = ob + (int64_t)(m0 + r) * n + n0 + lane;
+    if (psum) v = v + psum[o];
+    if (v != v) v = u2f(0x7fc00000u);
+    store_from_f32<OUT>(dst, o, v);
+  }
+}
+
+template <uint32_t IN, int R>
+int launch_rows(uint32_t out, hipStream_t st, const void *lhs, const void *rhs, void *dst, const float *psum, int m,
+                int k, int n, int batch, int lt) {
+  const int row_tiles = (m + R - 1) / R;
+  const int64_t waves = (int64_t)row_tiles * ((n + 63) / 64);
+  const dim3 grid((unsigned)((waves + 3) / 4), 1, (unsigned)batch);
+  switch (out) {
+  case WAFER_FMT_F32:
+    hipLaunchKernelGGL((gemm_formal_rows_kernel<IN, WAFER_FMT_F32, R>), grid, dim3(256), 0, st, lhs, rhs, dst, psum, m,
+                       k, n, lt, row_tiles);
+    break;
+  case WAFER_FMT_BF16:
+    hipLaunchKernelGGL((gemm_formal_rows_kernel<IN, WAFER_FMT_BF16, R>), grid, dim3(256), 0, st, lhs, rhs, dst, psum,
+                       m, k, n, lt, row_tiles);
+    break;
+  default:
+    hipLaunchKernelGGL((gemm_formal_rows_kernel<IN, WAFER_FMT_F16, R>), grid, dim3(256), 0, st, lhs, rhs, dst, psum, m,
+                       k, n, lt, row_tiles);
+    break;
+  }
+  return launch_status("gemm_formal_rows_kernel");
+}
+
 template <uint32_t IN, int MT>
 int launch_out(uint32_t out, dim3 grid, hipStream_t st, const void *lhs, const void *rhs,
                void *dst, const float *psum, int m, int k, int n, int lt, int rt) {
@@ -157,6 +330,21 @@ int launch_out(uint32_t out, dim3 grid, hipStream_t st, const void *lhs, const v
 template <uint32_t IN>
 int launch_in(uint32_t out, int cus, hipStream_t st, const void *lhs, const void *rhs, void *dst,
               const float *psum, uint32_t m, uint32_t k, uint32_t n, uint32_t batch, int lt, int rt) {
+  // Normal rhs, chains in registers: the most rows per wave that still give
+  // (nearly) every SIMD a wave.  Fewer waves than that leave a wave's one chain
+  // waiting on its loads, where the tiled kernel is the faster one in F32 (us,
+  // tiled / 4 rows: 64 x 256 x 256 5.8 / 7.2, 128 x 2048 x 512 31 / 38); in
+  // 16 bits its widening of every operand twice costs more (16 x 300 x 700:
+  // 10.5 / 7.0 with one row).
+  if (!rt) {
+    auto waves = [&](uint64_t r) { return ((m + r - 1) / r) * ((n + 63) / 64) * batch; };
+    const uint64_t simds = 4 * (uint64_t)cus, most = simds * 7 / 8;
+    if (m > 4 && waves(8) >= most) return launch_rows<IN, 8>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+    if (m > 2 && waves(4) >= (IN == WAFER_FMT_F32 ? most : simds / 2))
+      return launch_rows<IN, 4>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+    if (IN == WAFER_FMT_F32 ? m <= 2 && waves(1) >= most : waves(1) <= simds)
+      return launch_rows<IN, 1>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+  }
   auto grid = [&](uint32_t t) { return (uint64_t)((n + t - 1) / t) * ((m + t - 1) / t) * batch; };
   if (grid(64) >= (uint64_t)cus)
     return launch_out<IN, 4>(out, dim3((n + 63) / 64, (m + 63) / 64, batch), st, lhs, rhs, dst, psum,
