@@ -503,3 +503,32 @@ def test_additive_mask_tails(hip, oracle, L):
         got = run_masked(hip, BF16, q, k, v, 0.125, **kw)
         attention_gate(tof(oracle, BF16, got), tof(oracle, BF16, ref), what="additive tail")
         assert not got[:, :, 4].any()
+
+
+@pytest.mark.parametrize("fmt", [F16, BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("Bn,Hq,Hkv,Sq,Skv", [(2, 96, 24, 130, 130), (1, 90, 90, 257, 257), (1, 52, 13, 577, 600),
+                                              (1, 256, 64, 129, 70), (1, 32, 8, 1025, 1025)])
+def test_causal_middle_block(hip, oracle, Bn, Hq, Hkv, Sq, Skv, fmt):
+    """Odd counts of query blocks (three up) on grids where the middle block
+    rides on pair 0, through the dense and the strided entry (bit-identical),
+    against float64 attention on some heads under the attention policy; the
+    rows of every block against the masked kernels' on all heads."""
+    say("middle block", Bn, Hq, Hkv, Sq, Skv, fmt)
+    g = torch.Generator(device="cuda").manual_seed(Sq + Hq)
+    dt = torch.float16 if fmt == F16 else torch.bfloat16
+    q, k, v = (torch.randn(Bn, h, s, 128, generator=g, device="cuda").to(dt)
+               for h, s in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    scale = 128 ** -0.5
+    o, om = torch.full_like(q, 7.0), torch.empty_like(q)
+    hip.attention_prefill(q, k, v, o, scale, causal=True, fmt=fmt)
+    hip.attention_prefill_masked(q, k, v, om, scale, causal=True, fmt=fmt)
+    attention_gate(o.float().cpu().numpy(), om.float().cpu().numpy(), what="against the masked kernel")
+    for h in (0, Hq // 2, Hq - 1):
+        x = q[-1, h].double() @ k[-1, h // (Hq // Hkv)].double().t() * scale
+        x.masked_fill_(torch.from_numpy(~band(Sq, Skv, 0)).cuda(), float("-inf"))
+        ref = torch.softmax(x, dim=-1) @ v[-1, h // (Hq // Hkv)].double()
+        attention_gate(o[-1, h].float().cpu().numpy(), ref.float().cpu().numpy(), what=f"head {h}")
+    vt = v.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3)
+    ot = torch.full((Bn, Sq, Hq, 128), 7.0, dtype=dt, device="cuda").permute(0, 2, 1, 3)
+    hip.attention_prefill_strided(q, k, vt, ot, scale, causal=True, fmt=fmt)
+    assert torch.equal(ot.contiguous().view(torch.int16), o.view(torch.int16))

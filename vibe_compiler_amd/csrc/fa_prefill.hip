@@ -154,7 +154,10 @@ __device__ inline f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
 
-template <typename T, bool CAUSAL, bool STRIDED = false>
+// MID (causal, an odd count of query blocks above one): the middle block, which
+// would be a workgroup of its own with its early waves idle, follows block 0
+// on the early waves of pair 0, whose own block ends with the first key block.
+template <typename T, bool CAUSAL, bool STRIDED = false, bool MID = false>
 __global__ __launch_bounds__(THREADS) void fa_prefill_d128(
     const uint16_t *__restrict__ Q, const uint16_t *__restrict__ K,
     const uint16_t *__restrict__ V, uint16_t *__restrict__ O, int q_heads, int kv_heads,
@@ -510,14 +513,19 @@ __global__ __launch_bounds__(THREADS) void fa_prefill_d128(
     // (within each 16-lane group, lane i receives element i%4 of the
     // 4-element vectors at the addresses of lanes 4e + i/4, e = 0..3).
     const int l16 = lane & 15, g = lane >> 4;
-    const int q0 = qb_b * QB + (wave - 4) * 16;
+    int q0 = qb_b * QB + (wave - 4) * 16, nk_e = nk_b, nit_e = nite;
     // Q^T as the MFMA B operand: lane holds query l16, d = 32 s + 8 g + [0,8)
     u32x4 qreg[4];
-    {
-      const int row = min(q0 + l16, q_len - 1);
+    auto load_q = [&](u32x4 (&q)[4], int first) __attribute__((always_inline)) {
+      const int row = min(first + l16, q_len - 1);
 #pragma unroll
-      for (int s = 0; s < 4; ++s) qreg[s] = *(const u32x4 *)(Qp + (size_t)row * q_rs + s * 32 + g * 8);
-    }
+      for (int s = 0; s < 4; ++s) q[s] = *(const u32x4 *)(Qp + (size_t)row * q_rs + s * 32 + g * 8);
+    };
+    load_q(qreg, q0);
+    const int mid = n_qblocks / 2;  // MID: the middle block, after block 0
+    const bool more = MID && pair == 0;
+    u32x4 qmid[4];
+    if (more) load_q(qmid, mid * QB + (wave - 4) * 16);
     // LDS read offsets (bytes within a 16 KiB block), per lane:
     //  K (A operand, k-step s, key tile kt): row kt*16 + l16, chunk 4 s + g,
     //    swz = l16  ->  k_off[s] + kt * 4096
@@ -640,23 +648,42 @@ __global__ __launch_bounds__(THREADS) void fa_prefill_d128(
       }
     };
     auto nop = [&]() __attribute__((always_inline)) {};
+    auto finalize = [&]() __attribute__((always_inline)) {
+      // coefficient = Recip(l) (0 for an empty row), out = T(acc * coef)
+      const float l = xor16_sum(xor32_sum(l_part));
+      const float coef = (l == 0.0f) ? 0.0f : 1.0f / l;
+      uint16_t *orow = Op + (int64_t)(q0 + l16) * o_rs + 4 * g;
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        u32x2 packed;
+        packed[0] = narrow_pair<T>(acc_o[dt][0] * coef, acc_o[dt][1] * coef);
+        packed[1] = narrow_pair<T>(acc_o[dt][2] * coef, acc_o[dt][3] * coef);
+        if (q0 + l16 < q_len) *(u32x2 *)(orow + dt * 16) = packed;
+      }
+    };
 
     run([&](int t, auto slot, auto &&kdma, auto &&vdma) __attribute__((always_inline)) {
       constexpr int P = decltype(slot)::value;
-      if (t < nite) {
+      if (t < nit_e) {
         compute(2 * t, (const char *)sbuf[P][0], (const char *)sbuf[P][2], kdma, vdma);
-        if (2 * t + 1 < nk_b) compute(2 * t + 1, (const char *)sbuf[P][1], (const char *)sbuf[P][3], nop, nop);
-        if (t == nite - 1) {
-          // finalize: coefficient = Recip(l) (0 for an empty row), out = T(acc * coef)
-          const float l = xor16_sum(xor32_sum(l_part));
-          const float coef = (l == 0.0f) ? 0.0f : 1.0f / l;
-          uint16_t *orow = Op + (int64_t)(q0 + l16) * o_rs + 4 * g;
+        if (2 * t + 1 < nk_e) compute(2 * t + 1, (const char *)sbuf[P][1], (const char *)sbuf[P][3], nop, nop);
+        if (t == nit_e - 1) finalize();
+        if constexpr (MID && P == 0) {
+          if (more && t == 0) {  // block 0 is done (one key block): on to the middle block, same stage
+            q0 = mid * QB + (wave - 4) * 16;
+            nk_e = min(kv_blocks, mid + 1);
+            nit_e = (nk_e + 1) / 2;
+            mc_ref = NOREF;
+            l_part = 0.0f;
 #pragma unroll
-          for (int dt = 0; dt < 8; ++dt) {
-            u32x2 packed;
-            packed[0] = narrow_pair<T>(acc_o[dt][0] * coef, acc_o[dt][1] * coef);
-            packed[1] = narrow_pair<T>(acc_o[dt][2] * coef, acc_o[dt][3] * coef);
-            if (q0 + l16 < q_len) *(u32x2 *)(orow + dt * 16) = packed;
+            for (int s = 0; s < 4; ++s) qreg[s] = qmid[s];
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+              for (int j = 0; j < 4; ++j) acc_o[dt][j] = 0.0f;
+            for (int kb = 0; kb < min(2, nk_e); ++kb)
+              compute(kb, (const char *)sbuf[P][kb], (const char *)sbuf[P][2 + kb], nop, nop);
+            if (nit_e == 1) finalize();
           }
         }
       } else {
@@ -674,17 +701,28 @@ template <bool STRIDED>
 int launch_fa(wafer_hip_context *ctx, uint32_t format, bool causal, const void *q, const void *k, const void *v,
               void *o, uint32_t q_heads, uint32_t kv_heads, uint32_t q_len, uint32_t kv_len, float c, int bh_count,
               int n_qblocks, const FaStrides &st) {
-  dim3 grid((unsigned)(bh_count * ((n_qblocks + 1) / 2)));  // one workgroup per pair of query blocks
-#define FA_GO(T, CZ)                                                                                           \
-  hipLaunchKernelGGL((fa_prefill_d128<T, CZ, STRIDED>), grid, dim3(THREADS), 0, ctx->stream, (const uint16_t *)q, \
+  // One workgroup per pair of query blocks, one workgroup per CU.  The middle
+  // block of an odd count rides on pair 0 (causal) where its own workgroups
+  // would start another round (us: 32 heads x 1025 26.2 -> 23.0, 28 x 1200 28.1
+  // -> 24.9, 4 x 32 x 300 17.4 -> 14.4; 28 x 4000, no round less, 157 against
+  // 158).
+  const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  auto rounds = [&](int64_t pairs) { return (bh_count * pairs + cus - 1) / cus; };
+  const bool mid = causal && n_qblocks % 2 == 1 && n_qblocks > 1 &&
+                   rounds(n_qblocks / 2) < rounds((n_qblocks + 1) / 2);
+  dim3 grid((unsigned)(bh_count * ((n_qblocks + (mid ? 0 : 1)) / 2)));
+#define FA_GO(T, CZ, MZ)                                                                                       \
+  hipLaunchKernelGGL((fa_prefill_d128<T, CZ, STRIDED, MZ>), grid, dim3(THREADS), 0, ctx->stream, (const uint16_t *)q, \
                      (const uint16_t *)k, (const uint16_t *)v, (uint16_t *)o, (int)q_heads, (int)kv_heads,      \
                      (int)q_len, (int)kv_len, c, bh_count, n_qblocks, st)
   if (format == WAFER_FMT_BF16) {
-    if (causal) FA_GO(__bf16, true);
-    else FA_GO(__bf16, false);
+    if (mid) FA_GO(__bf16, true, true);
+    else if (causal) FA_GO(__bf16, true, false);
+    else FA_GO(__bf16, false, false);
   } else {
-    if (causal) FA_GO(_Float16, true);
-    else FA_GO(_Float16, false);
+    if (mid) FA_GO(_Float16, true, true);
+    else if (causal) FA_GO(_Float16, true, false);
+    else FA_GO(_Float16, false, false);
   }
 #undef FA_GO
   return launch_status("fa_prefill_d128");
