@@ -46,11 +46,12 @@ def _check(got, a, b, half_ulp):
 
 ROWS = [(1, 128, 4096, 3), (15, 130, 96, 2), (16, 16, 32, 3), (17, 4096, 160, 3), (31, 33, 8192, 2), (32, 8192, 96, 3),
         (33, 1000, 544, 2), (48, 10272, 64, 3), (63, 20, 2080, 3), (64, 12288, 128, 2), (64, 640, 1024, 3)]
-# tiles of the 4-wave kernel whose last row / column of tiles is shifted back
-# to the edge: 64x64, 64x128, 128x64, 128x128, 128x192 and 256x256, with n of
-# every alignment
-TILES = [(65, 64, 128, 3), (127, 72, 256, 2), (100, 16400, 128, 3), (129, 130, 192, 2), (300, 4100, 128, 3),
-         (300, 6145, 256, 2), (1000, 6148, 128, 3), (300, 28648, 64, 2), (300, 28656, 128, 3), (130, 60, 256, 3)]
+# few outputs of more rows (64 x 32 tiles, SwiGLU 64 x 64), and tiles of the
+# 4-wave kernel whose last row / column of tiles is shifted back to the edge:
+# 64x64, 64x128, 128x64, 128x128, 128x192 and 256x256, with n of every alignment
+TILES = [(200, 4100, 128, 3), (65, 64, 128, 3), (127, 72, 256, 2), (100, 16400, 128, 3), (129, 130, 192, 2), (300, 4100, 128, 3),
+         (300, 6145, 256, 2), (1000, 6148, 128, 3), (300, 28648, 64, 2), (300, 28656, 128, 3), (130, 60, 256, 3),
+         (1000, 500, 96, 2), (120, 4096, 2080, 3)]
 
 
 @pytest.mark.parametrize("m,n,k,fmt", ROWS + TILES)

@@ -47,9 +47,10 @@ struct GemmArgs {
   float *part;
 };
 
-// Few-row GEMMs (gemm_skinny.hip): true where the weight-streaming kernel
-// serves a product of m rows, and its launch.
-bool gemm_is_skinny(int m);
+// GEMMs of few rows or few outputs (gemm_skinny.hip): true where the weight-
+// streaming kernel serves a product of m x n (of one of the two products of a
+// SwiGLU, so that it sums as the two plain calls do), and its launch.
+bool gemm_is_skinny(int m, int n, int cus);
 template <int KIND, int OUT> int launch_gemm_skinny(hipStream_t st, GemmArgs args, int cus);
 
 }  // namespace wafer

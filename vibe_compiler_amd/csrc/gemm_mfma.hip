@@ -677,8 +677,8 @@ gemm_nt_kernel(GemmArgs args) {
 // the tile before it does not.
 //
 // Measured on cold weights against the 8-wave kernel's 128- and 256-row tiles
-// that served these shapes (us, bits unchanged): 128 x 4096, K 4096 36.8 ->
-// 21.0 (64x64), 300 x 6144 37.5 -> 31.3 (64x128), 300 x 4096 32.6 -> 27.7
+// that served these shapes (us, bits unchanged): 200 x 4096, K 4096 32.9 ->
+// 21.2 (64x64), 300 x 6144 37.5 -> 31.3 (64x128), 300 x 4096 32.6 -> 27.7
 // (128x64), 777 x 6144 69.8 -> 54.6 (128x192), SwiGLU 128 x 28672 119.4 -> 59.4
 // (128x128), SwiGLU 777 x 28672 243.6 -> 215.1 (256x256).
 template <int KIND, int OUT, int BM, int BN, int SB = 64, int WM = 2, int WN = 2, bool SPLIT = false,
@@ -1002,7 +1002,7 @@ constexpr TileCost TILES[] = {{256, 256, 1250, 6000}, {256, 224, 1200, 6000}, {1
 // The tile for m x n outputs (-1: none, the product is narrower than every
 // tile).  256x224 tiles serve SwiGLU products that they divide.  Examples at
 // K 4096: (1024, 6144) 128x192, (1024, 4096) 128x128, (300, 4096) 128x64,
-// (300, 6144) 64x128, (128, 4096) 64x64.
+// (300, 6144) 64x128, (200, 4096) 64x64.
 int pick_tile(int m, int n, int kbytes, bool swiglu, int cus, long *ns) {
   int best = -1;
   for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
@@ -1113,8 +1113,9 @@ int plan_split(int m, int n, int kbytes, int cus) {
 // Sets up args.ksplit / args.part for a 16-bit GEMM (growing the context's
 // partial-tile area when a split is planned).
 int prepare_split(wafer_hip_context *ctx, GemmArgs &args) {
-  if (gemm_is_skinny(args.m)) return WAFER_HIP_OK;
-  const int s = plan_split(args.m, args.n, args.kbytes, ctx->cu_count > 0 ? ctx->cu_count : 256);
+  const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  if (gemm_is_skinny(args.m, args.n, cus)) return WAFER_HIP_OK;
+  const int s = plan_split(args.m, args.n, args.kbytes, cus);
   if (s < 2) return WAFER_HIP_OK;
   WAFER_TRY(ensure_workspace(ctx, &ctx->partials, &ctx->partials_bytes, (size_t)s * args.m * args.n * sizeof(float)));
   args.ksplit = s;
@@ -1126,7 +1127,8 @@ template <int KIND, int OUT>
 int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
   const hipStream_t st = ctx->stream;
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  if (gemm_is_skinny(args.m)) return launch_gemm_skinny<KIND, OUT>(st, args, cus);
+  if (gemm_is_skinny(args.m, OUT == OUT_SWIGLU ? args.n / 2 : args.n, cus))
+    return launch_gemm_skinny<KIND, OUT>(st, args, cus);
   if constexpr (KIND != KIND_I8 && OUT != OUT_SWIGLU) {
     if (args.ksplit > 1) {  // planned by the entry (prepare_split)
       args.tiles_m = args.m / 256;

@@ -1,5 +1,5 @@
 // gemm_skinny.hip -- MFMA GEMMs of few rows (decode steps, short prompts):
-// y [m, n] = a [m, K] . bt [n, K]^T with m at most SKINNY_ROWS, bf16 / f16
+// y [m, n] = a [m, K] . bt [n, K]^T with m at most 64, or few outputs, bf16 / f16
 // (f32 accumulate) and int8 (exact int32 accumulate).
 //
 // What bounds it is the weight bt, read once from HBM, and then the
@@ -29,6 +29,14 @@
 //
 // The order of the sum of one output depends on K alone (not on m, n, or the
 // epilogue), so the fused epilogues keep the bits of the unfused calls.
+//
+// More rows on few columns take the same kernel on tiles of 64 x 32 (SwiGLU: 64 x
+// 64, the two products' columns), wherever those are one round of workgroups at
+// most: twice the workgroups of 64 x 64 tiles and rings three units deep, so more
+// bytes in flight on more CUs, and no stage barrier (64 x 64 tiles here were no
+// faster than the tile kernel's).  Against that kernel (us): 128 x 4096, K 4096
+// 21.0 -> 16.3; 128 x 4096 with residual, K 14336 74 -> 52; int8 300 x 1389, K
+// 3520 21.8 -> 11.5; 256 x 2048, K 1024 6.9 -> 6.0.
 //
 // Rows past m, columns past n and K past its end read as zero (buffer range)
 // and are not stored.
@@ -77,13 +85,14 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_nt_skinny_kernel(GemmA
   __shared__ __align__(1024) uint8_t lds[W * D * SLOT];
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = blockIdx.x * (16 * NT);
+  const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
   const int kb = args.kbytes;
   const int units = (kb + 127) / 128, iters = (units + W - 1) / W;
 
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
       (void *)(args.bt + (size_t)n0 * kb), 0, min(16 * NT, args.n - n0) * kb, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)args.a, 0, args.m * kb, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)(args.a + (size_t)m0 * kb), 0, min(16 * MT, args.m - m0) * kb, 0x00020000);
 
   // One DMA instruction moves 8 rows x 128 bytes: lane l fills chunk position
   // l % 8 of row l / 8, so it loads the chunk that the swizzle (chunk ^ (row
@@ -166,7 +175,7 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_nt_skinny_kernel(GemmA
     for (int j = 0; j < NT; ++j) part[wv][i * NT + j][lane] = acc[i][j];
   __syncthreads();
 
-  // the fold: lane (l16, g) of a tile holds row 16 i + l16, columns
+  // the fold: lane (l16, g) of a tile holds row m0 + 16 i + l16, columns
   // n0 + 16 j + 4 g .. +3
   auto fold = [&](int tile, int ln) __attribute__((always_inline)) {
     acc_t s = part[0][tile][ln];
@@ -184,7 +193,7 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_nt_skinny_kernel(GemmA
     const bool vec = nf % 4 == 0 && ((uintptr_t)args.y & 7) == 0;
     for (int q = threadIdx.x; q < TILES / 2 * 64; q += 64 * W) {
       const int t = q >> 6, ln = q & 63;  // pair t: row tile t / (NT / 2), column tiles 2 (t % (NT / 2)), + 1
-      const int row = 16 * (t / (NT / 2)) + (ln & 15), f0 = n0 / 2 + 16 * (t % (NT / 2)) + 4 * (ln >> 4);
+      const int row = m0 + 16 * (t / (NT / 2)) + (ln & 15), f0 = n0 / 2 + 16 * (t % (NT / 2)) + 4 * (ln >> 4);
       if (row >= args.m || f0 >= nf) continue;
       const acc_t gt = fold(2 * t, ln), up = fold(2 * t + 1, ln);
       uint16_t o[4];
@@ -207,7 +216,7 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_nt_skinny_kernel(GemmA
                      (OUT != OUT_NARROW_RES || ((uintptr_t)args.res & 7) == 0);
     for (int q = threadIdx.x; q < TILES * 64; q += 64 * W) {
       const int t = q >> 6, ln = q & 63;
-      const int row = 16 * (t / NT) + (ln & 15), col = n0 + 16 * (t % NT) + 4 * (ln >> 4);
+      const int row = m0 + 16 * (t / NT) + (ln & 15), col = n0 + 16 * (t % NT) + 4 * (ln >> 4);
       if (row >= args.m || col >= args.n) continue;
       const acc_t s = fold(t, ln);
       const size_t o = (size_t)row * args.n + col;
@@ -273,10 +282,11 @@ constexpr int ring_depth(int mt, int nt) {
   return d > 8 ? 8 : d < 2 ? 2 : d;
 }
 
-template <int KIND, int OUT, int MT, int NT>
+template <int KIND, int OUT, int MT, int NT, int D = ring_depth(MT, NT)>
 int launch_cols(hipStream_t st, const GemmArgs &args) {
-  hipLaunchKernelGGL((gemm_nt_skinny_kernel<KIND, OUT, MT, NT, ring_depth(MT, NT)>),
-                     dim3((unsigned)((args.n + 16 * NT - 1) / (16 * NT))), dim3(64 * SKINNY_WAVES), 0, st, args);
+  hipLaunchKernelGGL((gemm_nt_skinny_kernel<KIND, OUT, MT, NT, D>),
+                     dim3((unsigned)((args.n + 16 * NT - 1) / (16 * NT)), (unsigned)((args.m + 16 * MT - 1) / (16 * MT))),
+                     dim3(64 * SKINNY_WAVES), 0, st, args);
   return launch_status("gemm_nt_skinny_kernel");
 }
 
@@ -296,10 +306,14 @@ int launch_rows(hipStream_t st, const GemmArgs &args, int cus) {
 
 }  // namespace
 
-bool gemm_is_skinny(int m) { return m <= SKINNY_ROWS; }
+bool gemm_is_skinny(int m, int n, int cus) {
+  return m <= SKINNY_ROWS || (long)((m + 63) / 64) * ((n + 31) / 32) <= cus;
+}
 
 template <int KIND, int OUT>
 int launch_gemm_skinny(hipStream_t st, GemmArgs args, int cus) {
+  if (args.m > SKINNY_ROWS)
+    return launch_cols<KIND, OUT, 4, OUT == OUT_SWIGLU ? 4 : 2, OUT == OUT_SWIGLU ? 2 : 3>(st, args);
   if (args.m <= 16) return launch_rows<KIND, OUT, 1>(st, args, cus);
   if (args.m <= 32) return launch_rows<KIND, OUT, 2>(st, args, cus);
   return launch_rows<KIND, OUT, 4>(st, args, cus);
