@@ -75,7 +75,8 @@ typedef struct wafer_hip_context wafer_hip_context;
  * and never shrunk -- the split-K partial tiles of the MFMA GEMMs (up to
  * 4 * m * n * 4 bytes for the 16-bit GEMMs, 64 MiB at the decoder layer's
  * down projection), the re-laid-out [n,k] rhs of a Normal-orientation GEMM
- * (k * n * element bytes) and FD's chunk states for small batches.  Growing
+ * (k * n * element bytes) and FD's chunk states for small batches (4.1 MiB at
+ * least).  Growing
  * is refused on a capturing stream, so a caller that captures runs each
  * shape once eagerly first.  A grown area's old buffer is kept until
  * wafer_hip_context_destroy, so graphs captured before a later, larger eager
@@ -137,7 +138,7 @@ int wafer_hip_gemm(wafer_hip_context *ctx, const void *lhs, const void *rhs,
  * out_format F32 or the input format.  Any m, n; k a multiple of 32 (64-byte
  * K stages); other k return WAFER_HIP_E_UNSUPPORTED.  Long-K shapes whose
  * 128x128 grid is at most one round of workgroups (k * 2 >= 16384 bytes, m
- * and n multiples of 256) split K over 4 workgroups with f32 partials in a
+ * and n multiples of 256) may split K over 4 workgroups with f32 partials in a
  * context-owned area (4 * m * n * 4 bytes, grown on first use; growing is
  * refused on a capturing stream, so a caller that captures runs the shape
  * once eagerly first).  Results repeat bit for bit for a given shape. */
