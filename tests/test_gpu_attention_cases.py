@@ -486,6 +486,63 @@ def test_boolean_masks(hip, oracle, D, Sq, L):
     assert np.array_equal(ones, run_masked(hip, F16, q, k, v, scale))
 
 
+@pytest.mark.parametrize("fmt", [F16, BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("D", [16, 64, 128])
+@pytest.mark.parametrize("sign", [1, -1], ids=["positive", "negative"])
+def test_far_scores_under_window_and_boolean_masks(hip, oracle, fmt, D, sign):
+    """Scores so large that float32 holds no fraction of them (and, negative in
+    BF16 at scale 4, finite scores t whose t * log2(e) overflows), under a
+    window and under boolean masks, at references far on either side and
+    leaving one (a window that grows): the softmax is 1 at the largest visible
+    score (two ties share it evenly), so a row is that V row, or the mean of the
+    tied ones, which the format holds exactly here, bit for bit."""
+    say("far scores", fmt, D, sign)
+    rng = np.random.default_rng(D + fmt + sign)
+    dt = torch.float16 if fmt == F16 else torch.bfloat16
+    Sq, L = 100, 200 if fmt == F16 else 128
+    # score of key j: sign * 2^27 .. 2^30 (F16), 2^125 .. 2^126 (BF16), times the scale
+    unit = [(2.0 ** 14, 2.0 ** 13), (2.0 ** 15, 2.0 ** 15)] if fmt == F16 else [(2.0 ** 61, 2.0 ** 64)]
+    bits = 10 if fmt == F16 else 7
+    mant = 1 + rng.permutation(2 ** bits)[:L] / 2 ** bits
+    top = int(np.argmax(sign * mant))  # goes to keys 63 and 64, across a block boundary
+    mant[[63, top]] = mant[[top, 63]]
+    mant[64] = mant[63]
+    for a, b in unit:
+        for scale in (0.125, 1.0, 8.0) if fmt == F16 else (0.125, 1.0, 4.0 if sign < 0 else 1.5):
+            q, k = torch.zeros(1, 1, Sq, D, dtype=dt), torch.zeros(1, 1, L, D, dtype=dt)
+            q[..., 0] = a * sign
+            k[..., 0] = torch.from_numpy(mant * b).to(dt)
+            v = torch.from_numpy(rng.integers(-8, 9, (1, 1, L, D))).to(dt)
+            qn, kn, vn = (x.view(torch.int16).numpy().view(np.uint16) for x in (q, k, v))
+            t = (q[0, 0, :1, 0].float() * k[0, 0, :, 0].float()) * scale
+            t = t.numpy()
+            assert np.isfinite(t).all()
+            keep = np.zeros((1, 1, 1, L), np.uint8)
+            keep[..., rng.permutation(L)[:90]] = 1
+            both = keep.copy()
+            both[..., 63:65] = 1
+            one = np.zeros((1, 1, 1, L), np.uint8)
+            one[..., int(np.argmin(t))] = 1
+            cases = [dict(causal=True, diagonal=L - Sq, window=1), dict(causal=True, diagonal=L - Sq, window=70),
+                     dict(keep=keep), dict(keep=both), dict(keep=one),
+                     dict(keep=np.broadcast_to(both, (1, 1, Sq, L)).copy())]
+            for kw in cases:
+                vis = np.broadcast_to(kw.get("keep", 1) != 0, (1, 1, Sq, L))[0, 0].copy()
+                if kw.get("causal"):
+                    vis &= band(Sq, L, kw["diagonal"], kw["window"])
+                x = np.where(vis, t[None], -np.inf)
+                hit = x == x.max(axis=1, keepdims=True)
+                got = tof(oracle, fmt, run_masked(hip, fmt, qn, kn, vn, scale, **kw))[0, 0]
+                ref = hit.astype(np.float64) @ v[0, 0].double().numpy() / hit.sum(axis=1, keepdims=True)
+                assert hit.sum(axis=1).max() <= 2 and np.array_equal(got, ref), (a, b, scale, list(kw))
+    # a far negative reference left for a near one: the last key's score is 0
+    k[..., -1, :] = 0
+    got = tof(oracle, fmt, run_masked(hip, fmt, qn, k.view(torch.int16).numpy().view(np.uint16), vn, scale,
+                                      keep=np.ones((1, 1, 1, L), np.uint8)))[0, 0]
+    if sign < 0:
+        assert np.array_equal(got, np.broadcast_to(v[0, 0, -1].double().numpy(), got.shape))
+
+
 @pytest.mark.parametrize("L", [1, 2, 65, 191])
 def test_additive_mask_tails(hip, oracle, L):
     """An additive mask per query whose rows end inside a 64-key block, with

@@ -72,6 +72,7 @@ constexpr float RESCALE_BOUND = 256.0f;
 // until a score exceeds NOREF + 8, which sends the wave to the exact update).
 constexpr float NOREF = -0x1.fffffep127f;
 constexpr float LOG2E = 0x1.715476p+0f;
+constexpr float FAR_REF = 0x1p24f;  // MASK_SELECT: references past it are left to far_rows
 
 enum { MASK_CAUSAL = 1, MASK_GENERAL = 2, MASK_SELECT = 3 };
 constexpr uint32_t F_CAUSAL = WAFER_HIP_ATT_CAUSAL, F_WINDOW = WAFER_HIP_ATT_WINDOW,
@@ -135,6 +136,76 @@ __device__ inline float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Rows that the raw scores of MASK_SELECT do not serve, a row per four lanes,
+// straight from global memory.  The exponent fma(s, c, -round(max * c)) carries
+// the rounding of its reference, up to half an ulp, into every P: a factor of
+// 2^+-8 at 2^28, past F16's range from 2^29.  And where c > 1 a finite t = s *
+// scale past 2.36e38 overflows.  Here the maximum is subtracted from t
+// itself, as the reference does.  Rare, so small rather than fast, and judged
+// after the merge: told apart inside the pipelined loop it cost calls without
+// such a row 10 to 25 %, judged there up to 6 % at head_dim 128 and up to 10 %
+// for masks per query at head_dim 64 (32 heads x 2048: 104 -> 113 us).
+template <typename T, int D>
+__device__ inline void far_rows(const FaArgs &a, int bh, int qb, uint64_t rows) {
+  const int quad = threadIdx.x & 3, row = (threadIdx.x >> 2) & 63, i = qb * QB + row;
+  if (((rows >> row) & 1) == 0 || i >= a.q_len) return;  // all four lanes of a row alike
+  const int b = bh / a.q_heads, h = bh - b * a.q_heads;
+  const size_t kv = (size_t)(b * a.kv_heads + h / (a.q_heads / a.kv_heads)) * a.kv_cap * D;
+  const uint16_t *Kp = a.k + kv, *Vp = a.v + kv;
+  const uint16_t *q = a.q + ((size_t)bh * a.q_len + i) * D;
+  const uint8_t *keep = a.keep ? a.keep + b * a.keep_sb + h * a.keep_sh + i * a.keep_sq : nullptr;
+  const int lo = (a.flags & F_WINDOW) ? max(0, i + a.lo_off) : 0;
+  const int hi = (a.flags & F_CAUSAL) ? min(a.kv_len - 1, i + a.diag) : a.kv_len - 1;
+  auto score = [&](int key) -> float {
+    if (key > hi || (keep && keep[key] == 0)) return -__builtin_inff();
+    const uint16_t *k = Kp + (size_t)key * D;
+    float dot = 0.0f;
+#pragma unroll 1
+    for (int d = 0; d < D; ++d) dot = __builtin_fmaf(load_elem<T>(q + d), load_elem<T>(k + d), dot);
+    return dot * a.scale;
+  };
+  float m = -__builtin_inff();
+  bool nan = false;
+#pragma unroll 1
+  for (int key = lo + quad; key <= hi; key += 4) {
+    const float t = score(key);
+    nan = nan || t != t;
+    if (nan) break;  // the row is NaN whatever follows
+    m = fmaxf(m, t);
+  }
+  nan = __shfl_xor((int)nan, 1) || nan;
+  nan = __shfl_xor((int)nan, 2) || nan;
+  uint16_t *o = a.o + ((size_t)bh * a.q_len + i) * D + quad * (D / 4);
+  if (nan) {
+#pragma unroll 1
+    for (int d = 0; d < D / 4; ++d) o[d] = __builtin_bit_cast(uint16_t, (T)__builtin_nanf(""));
+    return;
+  }
+  m = fmaxf(m, __shfl_xor(m, 1));
+  m = fmaxf(m, __shfl_xor(m, 2));
+  if (m == -__builtin_inff()) m = 0.0f;  // no visible key: P = 0
+  float l = 0.0f, acc[D / 4];  // lane `quad` keeps d = quad D / 4 + [0, D / 4)
+#pragma unroll
+  for (int d = 0; d < D / 4; ++d) acc[d] = 0.0f;
+#pragma unroll 1
+  for (int k0 = lo; k0 <= hi; k0 += 4) {
+    const float t = score(k0 + quad);
+#pragma unroll 1
+    for (int n = 0; n < 4 && k0 + n <= hi; ++n) {
+      const float tn = __shfl(t, (threadIdx.x & 60) + n);
+      if (tn == -__builtin_inff()) continue;  // excluded
+      const float pn = __builtin_amdgcn_exp2f((tn - m) * LOG2E);
+      l += pn;
+      const uint16_t *v = Vp + (size_t)(k0 + n) * D + quad * (D / 4);
+#pragma unroll
+      for (int d = 0; d < D / 4; ++d) acc[d] = __builtin_fmaf(round_to<T>(pn), load_elem<T>(v + d), acc[d]);
+    }
+  }
+  const float coef = l == 0.0f ? 0.0f : 1.0f / l;
+#pragma unroll
+  for (int d = 0; d < D / 4; ++d) o[d] = __builtin_bit_cast(uint16_t, (T)f32_rounded(acc[d] * coef));
+}
+
 // One score through the score region and the masks: visible -> u = t*log2(e)
 // (a finite t whose u overflows is clamped to the lowest finite float),
 // invisible -> -inf, whatever t is (an invisible key is excluded).  Selects
@@ -191,6 +262,8 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
   // read and waits for the moves only at the iteration's barrier
   __shared__ __align__(1024) char sk0[2 * BLK], sk1[2 * BLK], sv0[2 * BLK], sv1[2 * BLK];
   __shared__ float sml[4][2][64];
+  // MASK_SELECT: by wave and phase, the queries (bit l32) left to far_rows
+  __shared__ uint32_t sfar[4][MASK == MASK_SELECT ? 2 : 1];
   // a boolean mask that is the same for every query, one bit per key
   __shared__ uint32_t skeep[MASK == MASK_CAUSAL ? 1 : KEEP_BLOCKS * 2];
 
@@ -512,7 +585,7 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
 
   // ---- merge of the two key halves of a query tile (reduce-scatter) and
   // finalize: out = narrow(acc * Recip(l)), 0 for a row that saw no key
-  auto finish_h = [&](char *xch, auto half_c) __attribute__((always_inline)) {
+  auto finish_h = [&](char *xch, int phase, auto half_c) __attribute__((always_inline)) {
     constexpr int H = decltype(half_c)::value;  // == half: every acc index stays static
     const float l_full = xor32_sum(l_part);
     sml[wave][0][lane] = m_ref;
@@ -535,6 +608,13 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
     const float s0 = __builtin_amdgcn_exp2f(m_ref - em), s1 = __builtin_amdgcn_exp2f(m1 - em);
     const float l = l_full * s0 + l1 * s1;
     const float coef = l == 0.0f ? 0.0f : 1.0f / l;
+    if constexpr (MASK == MASK_SELECT) {
+      // a far reference; one that was left again, whose P may have overflowed
+      // (infinity * 0 in the accumulators); or, where c > 1, a row without
+      // weight, whose visible scores may have overflowed
+      const bool far = (__builtin_fabsf(m_ref) > FAR_REF) & (m_ref != NOREF);
+      sfar[wave][phase] = (uint32_t)__ballot(far | (acc[0][0] != acc[0][0]) | ((a.c > 1.0f) & (l == 0.0f)));
+    }
     const f32x4 *px = (const f32x4 *)(xch + pw * (DT / 2) * 16 * 64 * 4);
     const int qi = q0 + l32;
     uint16_t *orow = a.o + ((size_t)bh * a.q_len + min(qi, a.q_len - 1)) * D;
@@ -556,11 +636,11 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
     __syncthreads();  // exchange reads done before the slot is reused
     asm volatile("; fa merge tail %0" ::"n"(H));  // keeps the two copies apart
   };
-  auto finish = [&](char *xch) __attribute__((always_inline)) {
+  auto finish = [&](char *xch, int phase) __attribute__((always_inline)) {
     if (half == 0)
-      finish_h(xch, std::integral_constant<int, 0>{});
+      finish_h(xch, phase, std::integral_constant<int, 0>{});
     else
-      finish_h(xch, std::integral_constant<int, 1>{});
+      finish_h(xch, phase, std::integral_constant<int, 1>{});
   };
 
   // ---- the pipeline.  Global iteration t (phase A: t < ta, then phase B)
@@ -691,7 +771,7 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
   // tn iterations (the half with one block fewer idles through its last
   // iteration: all its scores masked, P = 0), then PV of the last P (zero
   // for that half) and the merge.
-  auto run_phase = [&](int qb, int lo, int tn, int nh, int &t) __attribute__((always_inline)) {
+  auto run_phase = [&](int phase, int qb, int lo, int tn, int nh, int &t) __attribute__((always_inline)) {
     load_q(qb);
     reset();
     if (nh > 0) load_mask(lo + half);
@@ -725,7 +805,7 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
       else
         run(std::integral_constant<int, 0>{});
     }
-    finish((t & 1) ? sv1 : sv0);  // both halves of the free V slot
+    finish((t & 1) ? sv1 : sv0, phase);  // both halves of the free V slot
   };
 
   if (niter > 0) {
@@ -735,8 +815,19 @@ __attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void 
     __syncthreads();
   }
   int t = 0;
-  run_phase(qb_a, lo_a, ta, na_h, t);
-  if (has_b) run_phase(qb_b, lo_b, tb, nb_h, t);
+  run_phase(0, qb_a, lo_a, ta, na_h, t);
+  if (has_b) run_phase(1, qb_b, lo_b, tb, nb_h, t);
+  if constexpr (MASK == MASK_SELECT) {  // (the merge's last barrier published sfar)
+    int id = blockIdx.x;
+    asm volatile("" : "+s"(id)::"memory");  // nothing of this is kept in registers over the loop above
+    const int pair2 = id / a.bh_count;
+    for (int phase = 0; phase < 2; ++phase) {
+      const int qb = phase ? pair2 : a.n_qblocks - 1 - pair2;
+      if (phase && (a.single || qb >= a.n_qblocks - 1 - pair2)) break;
+      const uint32_t r0 = sfar[0][phase] | sfar[2][phase], r1 = sfar[1][phase] | sfar[3][phase];
+      if (__builtin_expect(r0 | r1, 0)) far_rows<T, D>(a, id - pair2 * a.bh_count, qb, r0 | (uint64_t)r1 << 32);
+    }
+  }
 }
 
 // ---- the small-head_dim lane: one thread per query row
