@@ -327,23 +327,40 @@ int launch_out(uint32_t out, dim3 grid, hipStream_t st, const void *lhs, const v
   return launch_status("gemm_formal_kernel");
 }
 
+// Rows per wave of gemm_formal_rows_kernel where it serves a product, else 0.
+// Normal rhs, chains in registers: the most rows per wave that still give
+// (nearly) every SIMD a wave.  Fewer waves than that leave a wave's one chain
+// waiting on its loads, where the tiled kernel is the faster one in F32 (us,
+// tiled / 4 rows: 64 x 256 x 256 5.8 / 7.2, 128 x 2048 x 512 31 / 38); in
+// 16 bits its widening of every operand twice costs more (16 x 300 x 700:
+// 10.5 / 7.0 with one row).
+//
+// A transposed lhs costs the rows kernel one cache line per k and row tile
+// (the 16 lanes of a row stand a whole row of m apart), where the tiled kernel
+// reads it whole.  There it serves few rows, of which the tiles would be mostly
+// padding, and 16 bits over a k that pays for it (us, tiled / rows: F32 128 x
+// 8192, k 512 42.7 / 72.0, 256 x 300, k 1024, batch 8 67 / 134, but 16 x 8192, k
+// 512, batch 8 148 / 68; BF16 256 x 2048, k 16 5.3 / 6.8, k 128 11.5 / 14.7, but
+// k 512 and up 0.5 to 0.98 of the tiled time; F16 from k 48 on).
+int rows_per_wave(uint32_t in, uint64_t m, uint64_t k, uint64_t n, uint64_t batch, int lt, int rt, uint64_t cus) {
+  if (rt) return 0;
+  auto waves = [&](uint64_t r) { return ((m + r - 1) / r) * ((n + 63) / 64) * batch; };
+  const uint64_t simds = 4 * cus, most = simds * 7 / 8;
+  const bool f32 = in == WAFER_FMT_F32;
+  const bool any_m = !lt || (!f32 && k >= (in == WAFER_FMT_BF16 ? 512u : 48u));
+  if (m > 4 && waves(8) >= most) return any_m || m <= 32 ? 8 : 0;
+  if (m > 2 && waves(4) >= (f32 ? most : simds / 2)) return any_m || m <= (f32 ? 16 : 32) ? 4 : 0;
+  return (f32 ? m <= 2 && waves(1) >= most : waves(1) <= simds) ? 1 : 0;
+}
+
 template <uint32_t IN>
 int launch_in(uint32_t out, int cus, hipStream_t st, const void *lhs, const void *rhs, void *dst,
               const float *psum, uint32_t m, uint32_t k, uint32_t n, uint32_t batch, int lt, int rt) {
-  // Normal rhs, chains in registers: the most rows per wave that still give
-  // (nearly) every SIMD a wave.  Fewer waves than that leave a wave's one chain
-  // waiting on its loads, where the tiled kernel is the faster one in F32 (us,
-  // tiled / 4 rows: 64 x 256 x 256 5.8 / 7.2, 128 x 2048 x 512 31 / 38); in
-  // 16 bits its widening of every operand twice costs more (16 x 300 x 700:
-  // 10.5 / 7.0 with one row).
-  if (!rt) {
-    auto waves = [&](uint64_t r) { return ((m + r - 1) / r) * ((n + 63) / 64) * batch; };
-    const uint64_t simds = 4 * (uint64_t)cus, most = simds * 7 / 8;
-    if (m > 4 && waves(8) >= most) return launch_rows<IN, 8>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
-    if (m > 2 && waves(4) >= (IN == WAFER_FMT_F32 ? most : simds / 2))
-      return launch_rows<IN, 4>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
-    if (IN == WAFER_FMT_F32 ? m <= 2 && waves(1) >= most : waves(1) <= simds)
-      return launch_rows<IN, 1>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+  switch (rows_per_wave(IN, m, k, n, batch, lt, rt, (uint64_t)cus)) {
+  case 8: return launch_rows<IN, 8>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+  case 4: return launch_rows<IN, 4>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+  case 1: return launch_rows<IN, 1>(out, st, lhs, rhs, dst, psum, m, k, n, batch, lt);
+  default: break;
   }
   auto grid = [&](uint32_t t) { return (uint64_t)((n + t - 1) / t) * ((m + t - 1) / t) * batch; };
   if (grid(64) >= (uint64_t)cus)
@@ -360,6 +377,12 @@ int launch_in(uint32_t out, int cus, hipStream_t st, const void *lhs, const void
 }  // namespace wafer
 
 using namespace wafer;
+
+// For the dispatch tests, host only: rows_per_wave on a chip of `cus` CUs.
+extern "C" int wafer_internal_formal_rows(uint32_t in_format, uint32_t m, uint32_t k, uint32_t n, uint32_t batch,
+                                          int lhs_t, int rhs_t, uint32_t cus) {
+  return rows_per_wave(in_format, m, k, n, batch, lhs_t, rhs_t, cus);
+}
 
 extern "C" int wafer_hip_gemm(wafer_hip_context *ctx, const void *lhs, const void *rhs,
                               void *dst, const void *psum, uint32_t m, uint32_t k, uint32_t n,
