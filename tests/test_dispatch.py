@@ -5,6 +5,10 @@ import ctypes
 import pytest
 
 F16, BF16, F32 = 2, 3, 5
+# operand kinds, epilogues and kernels of the MFMA GEMMs (gemm_common.h, gemm_mfma.hip)
+K_BF16, K_F16, K_I8 = 0, 1, 2
+OUT_F32, OUT_NARROW, OUT_I8, OUT_SWIGLU, OUT_RES = range(5)
+STREAM, TILE4, WAVE8, SPLIT = range(4)
 
 
 @pytest.fixture(scope="module")
@@ -12,6 +16,13 @@ def lib():
     from vibe_compiler_amd import backend
 
     return backend.load()
+
+
+def gemm_route(lib, m, n, k, out=OUT_NARROW, kind=K_BF16, cus=256):
+    """(kernel, tile rows, tile columns, splits) of m x n outputs over k elements; n counts a SwiGLU's two products."""
+    r = (ctypes.c_int * 4)()
+    lib.wafer_internal_gemm_route(kind, out, m, n, k * (1 if kind == K_I8 else 2), cus, r)
+    return tuple(r)
 
 
 def formal_rows(lib, fmt, m, k, n, batch=1, lt=0, rt=0, cus=256):
@@ -31,3 +42,18 @@ def test_formal_rows_of_a_transposed_lhs(lib, fmt, m, k, n, batch, normal, trans
     assert formal_rows(lib, fmt, m, k, n, batch) == normal
     assert formal_rows(lib, fmt, m, k, n, batch, lt=1) == transposed
     assert formal_rows(lib, fmt, m, k, n, batch, rt=1) == formal_rows(lib, fmt, m, k, n, batch, lt=1, rt=1) == 0
+
+
+@pytest.mark.parametrize("m,features,k,route", [
+    (256, 5504, 14336, (TILE4, 128, 128, 1)), (2048, 1024, 14336, (TILE4, 128, 128, 1)),
+    (128, 16384, 12288, (TILE4, 128, 128, 1)), (256, 16384, 14336, (TILE4, 128, 128, 1)),
+    (300, 11008, 12288, (WAVE8, 256, 256, 1)), (777, 16384, 12288, (WAVE8, 256, 256, 1)),
+    (512, 11008, 10240, (WAVE8, 256, 256, 1)), (777, 11008, 14336, (TILE4, 256, 256, 1)),
+    (777, 14336, 4096, (TILE4, 256, 256, 1)), (1024, 14336, 4096, (TILE4, 256, 224, 1)),
+    (1024, 14336, 14336, (TILE4, 256, 224, 1)), (16, 14336, 4096, (STREAM, 0, 0, 1))])
+def test_swiglu_takes_the_tile_it_was_priced_on(lib, m, features, k, route):
+    """Past K 12288 a SwiGLU product keeps the 128x128 tiles that its cost names
+    (they went to the 8-wave kernel, which has 256x256 SwiGLU tiles only); 256x256
+    tiles take the 8-wave kernel over rows of 3 or 5 times a power of two bytes."""
+    for kind in (K_BF16, K_F16):
+        assert gemm_route(lib, m, 2 * features, k, OUT_SWIGLU, kind) == route

@@ -1019,73 +1019,6 @@ int pick_tile(int m, int n, int kbytes, bool swiglu, int cus, long *ns) {
   return best;
 }
 
-template <int KIND, int OUT, int BM, int BN, int WM = 2, int WN = 2>
-int launch_dma4(hipStream_t st, GemmArgs args) {
-  args.tiles_m = (args.m + BM - 1) / BM;
-  args.tiles_n = (args.n + BN - 1) / BN;
-  const dim3 grid(args.tiles_m * args.tiles_n);
-  if constexpr (BM * BN >= 128 * 128) {
-    if (args.m % BM == 0 && args.n % BN == 0) {
-      hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, BM, BN, 128, WM, WN>), grid, dim3(256), 0, st, args);
-      return launch_status("gemm_nt_dma4_kernel");
-    }
-  }
-  if constexpr (BN != 224)
-    hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, BM, BN, 128, WM, WN, false, true>), grid, dim3(256), 0, st,
-                       args);
-  return launch_status("gemm_nt_dma4_kernel");
-}
-
-// The 8-wave kernel: 64-byte K stages, products narrower than 64 columns,
-// int8 on 256x256 tiles, and 128x128 tiles over a very long K.
-template <int KIND, int OUT, int SB>
-int launch_wave8(hipStream_t st, GemmArgs args) {
-  const int side = OUT == OUT_SWIGLU || (args.m % 256 == 0 && args.n % 256 == 0 &&
-                                         (long)(args.m / 256) * (args.n / 256) >= 192) ? 256 : 128;
-  args.tiles_m = (args.m + side - 1) / side;
-  args.tiles_n = (args.n + side - 1) / side;
-  const dim3 grid(args.tiles_m * args.tiles_n);
-  const bool full = args.m % side == 0 && args.n % side == 0;
-  if (side == 256 && full) {
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, false, SB>), grid, dim3(512), 0, st, args);
-  } else if constexpr (OUT == OUT_SWIGLU) {
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, true, SB>), grid, dim3(512), 0, st, args);
-  } else if (full) {
-    // 4 x 2 waves (each 32 x 64) measured 2-3 % faster than 2 x 4 on 128x128
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, false, SB, 4, 2>), grid, dim3(512), 0, st, args);
-  } else {
-    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, true, SB, 4, 2>), grid, dim3(512), 0, st, args);
-  }
-  return launch_status("gemm_nt_kernel");
-}
-
-template <int KIND, int OUT>
-int launch_tile(hipStream_t st, GemmArgs args, int tile) {
-  const int bm = TILES[tile].bm, bn = TILES[tile].bn;
-  if constexpr (KIND == KIND_I8) {
-    // whole 256x256 tiles keep 8 waves (int8 4096^3: 65.3 us against 68.5)
-    if (bm == 256) {
-      if (args.m % 256 == 0 && args.n % 256 == 0) return launch_wave8<KIND, OUT, 128>(st, args);
-      return launch_dma4<KIND, OUT, 128, 128>(st, args);
-    }
-  } else {
-    if (bm == 256 && bn == 256) return launch_dma4<KIND, OUT, 256, 256>(st, args);
-  }
-  if constexpr (OUT == OUT_SWIGLU) {
-    if (bn == 224) return launch_dma4<KIND, OUT, 256, 224, 4, 1>(st, args);
-  }
-  if (bn == 192) return launch_dma4<KIND, OUT, 128, 192>(st, args);
-  // past K 12288 the 8-wave kernel serves 128x128 tiles (777 x 4096, K 14336:
-  // 127 us against 145; K 11008: 101 against 102; 900 x 4096, K 8192: 83
-  // against 72)
-  if (bm == 128 && bn == 128)
-    return args.kbytes >= 24576 ? launch_wave8<KIND, OUT, 128>(st, args)
-                                : launch_dma4<KIND, OUT, 128, 128>(st, args);
-  if (bm == 128) return launch_dma4<KIND, OUT, 128, 64, 4, 1>(st, args);
-  if (bn == 128) return launch_dma4<KIND, OUT, 64, 128>(st, args);
-  return launch_dma4<KIND, OUT, 64, 64>(st, args);
-}
-
 // Split-K plan for 16-bit GEMMs whose 128x128 grid is at most one round of
 // workgroups and whose K is long: 256x256 tiles on the 4-wave kernel (half
 // the operand bytes per FLOP of 128x128 tiles), each tile's K split over
@@ -1110,27 +1043,114 @@ int plan_split(int m, int n, int kbytes, int cus) {
   return 1;
 }
 
-// Sets up args.ksplit / args.part for a 16-bit GEMM (growing the context's
-// partial-tile area when a split is planned).
-int prepare_split(wafer_hip_context *ctx, GemmArgs &args) {
-  const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  if (gemm_is_skinny(args.m, args.n, cus)) return WAFER_HIP_OK;
-  const int s = plan_split(args.m, args.n, args.kbytes, cus);
-  if (s < 2) return WAFER_HIP_OK;
-  WAFER_TRY(ensure_workspace(ctx, &ctx->partials, &ctx->partials_bytes, (size_t)s * args.m * args.n * sizeof(float)));
-  args.ksplit = s;
-  args.part = (float *)ctx->partials;
-  return WAFER_HIP_OK;
+// Which kernel serves a product of m x n (n counts both products of a
+// SwiGLU), and on which tile; what is priced here is what is launched.
+enum { ROUTE_STREAM = 0, ROUTE_TILE4 = 1, ROUTE_WAVE8 = 2, ROUTE_SPLIT = 3 };
+struct GemmRoute { int kernel, bm, bn, ksplit; };
+
+GemmRoute gemm_route(int kind, int out, int m, int n, int kbytes, int cus) {
+  const bool swiglu = out == OUT_SWIGLU, i8 = kind == KIND_I8;
+  if (gemm_is_skinny(m, swiglu ? n / 2 : n, cus)) return {ROUTE_STREAM, 0, 0, 1};
+  if (!i8 && !swiglu) {
+    const int split = plan_split(m, n, kbytes, cus);
+    if (split > 1) return {ROUTE_SPLIT, 256, 256, split};
+  }
+  // the 8-wave kernel: 64-byte K stages, products narrower than 64 columns,
+  // int8 on whole 256x256 tiles (4096^3: 65.3 us against 68.5), and what follows
+  const int side = swiglu || (m % 256 == 0 && n % 256 == 0 && (long)(m / 256) * (n / 256) >= 192) ? 256 : 128;
+  const GemmRoute wave8 = {ROUTE_WAVE8, side, side, 1};
+  long ns = 0;
+  const int tile = kbytes % 128 == 0 ? pick_tile(m, n, kbytes, swiglu, cus, &ns) : -1;
+  if (tile < 0) return wave8;
+  GemmRoute r = {ROUTE_TILE4, TILES[tile].bm, TILES[tile].bn, 1};
+  if (i8 && r.bm == 256) {
+    if (m % 256 == 0 && n % 256 == 0) return wave8;
+    r.bm = r.bn = 128;
+  }
+  if (swiglu) {
+    // 256x256 tiles over a K row of 3 or 5 times a power of two bytes: the
+    // 4-wave kernel's time jumps there (300 x 2 * 11008, 4-wave / 8-wave us: K
+    // 11008 285 / 285, 12288 380 / 319, 13312 335 / 339, 14336 367 / 368, 20480 650 /
+    // 510; 777 rows: K 8192 375 / 427, 12288 728 / 656, 14336 700 / 765).  The
+    // 8-wave kernel has no smaller SwiGLU tile, and needs none (128x128 tiles,
+    // against 8-wave 256x256: 256 x 2 * 5504, K 14336 157 / 393, 128 x 2 * 16384, K
+    // 12288 202 / 335).
+    const int odd = kbytes / (kbytes & -kbytes);
+    if (r.bm == 256 && r.bn == 256 && (odd == 3 || odd == 5)) return wave8;
+  } else if (r.bm == 128 && r.bn == 128 && kbytes >= 24576) {
+    // past K 12288 the 8-wave kernel serves 128x128 tiles (777 x 4096, K 14336:
+    // 127 us against 145; K 11008: 101 against 102; 900 x 4096, K 8192: 83
+    // against 72)
+    return wave8;
+  }
+  return r;
 }
 
+template <int KIND, int OUT, int BM, int BN, int WM = 2, int WN = 2>
+int launch_dma4(hipStream_t st, GemmArgs args) {
+  args.tiles_m = (args.m + BM - 1) / BM;
+  args.tiles_n = (args.n + BN - 1) / BN;
+  const dim3 grid(args.tiles_m * args.tiles_n);
+  if constexpr (BM * BN >= 128 * 128) {
+    if (args.m % BM == 0 && args.n % BN == 0) {
+      hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, BM, BN, 128, WM, WN>), grid, dim3(256), 0, st, args);
+      return launch_status("gemm_nt_dma4_kernel");
+    }
+  }
+  if constexpr (BN != 224)
+    hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT, BM, BN, 128, WM, WN, false, true>), grid, dim3(256), 0, st,
+                       args);
+  return launch_status("gemm_nt_dma4_kernel");
+}
+
+template <int KIND, int OUT, int SB>
+int launch_wave8(hipStream_t st, GemmArgs args, int side) {
+  args.tiles_m = (args.m + side - 1) / side;
+  args.tiles_n = (args.n + side - 1) / side;
+  const dim3 grid(args.tiles_m * args.tiles_n);
+  const bool full = args.m % side == 0 && args.n % side == 0;
+  if (side == 256 && full) {
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, false, SB>), grid, dim3(512), 0, st, args);
+  } else if constexpr (OUT == OUT_SWIGLU) {
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 256, 256, OUT, true, SB>), grid, dim3(512), 0, st, args);
+  } else if (full) {
+    // 4 x 2 waves (each 32 x 64) measured 2-3 % faster than 2 x 4 on 128x128
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, false, SB, 4, 2>), grid, dim3(512), 0, st, args);
+  } else {
+    hipLaunchKernelGGL((gemm_nt_kernel<KIND, 128, 128, OUT, true, SB, 4, 2>), grid, dim3(512), 0, st, args);
+  }
+  return launch_status("gemm_nt_kernel");
+}
+
+template <int KIND, int OUT>
+int launch_tile4(hipStream_t st, GemmArgs args, int bm, int bn) {
+  if constexpr (KIND != KIND_I8) {
+    if (bm == 256 && bn == 256) return launch_dma4<KIND, OUT, 256, 256>(st, args);
+  }
+  if constexpr (OUT == OUT_SWIGLU) {
+    if (bn == 224) return launch_dma4<KIND, OUT, 256, 224, 4, 1>(st, args);
+  }
+  if (bn == 192) return launch_dma4<KIND, OUT, 128, 192>(st, args);
+  if (bm == 128 && bn == 128) return launch_dma4<KIND, OUT, 128, 128>(st, args);
+  if (bm == 128) return launch_dma4<KIND, OUT, 128, 64, 4, 1>(st, args);
+  if (bn == 128) return launch_dma4<KIND, OUT, 64, 128>(st, args);
+  return launch_dma4<KIND, OUT, 64, 64>(st, args);
+}
+
+// The route of a product and its launch (a split grows the context's
+// partial-tile area).
 template <int KIND, int OUT>
 int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
   const hipStream_t st = ctx->stream;
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  if (gemm_is_skinny(args.m, OUT == OUT_SWIGLU ? args.n / 2 : args.n, cus))
-    return launch_gemm_skinny<KIND, OUT>(st, args, cus);
+  const GemmRoute r = gemm_route(KIND, OUT, args.m, args.n, args.kbytes, cus);
+  if (r.kernel == ROUTE_STREAM) return launch_gemm_skinny<KIND, OUT>(st, args, cus);
   if constexpr (KIND != KIND_I8 && OUT != OUT_SWIGLU) {
-    if (args.ksplit > 1) {  // planned by the entry (prepare_split)
+    if (r.kernel == ROUTE_SPLIT) {
+      WAFER_TRY(ensure_workspace(ctx, &ctx->partials, &ctx->partials_bytes,
+                                 (size_t)r.ksplit * args.m * args.n * sizeof(float)));
+      args.ksplit = r.ksplit;
+      args.part = (float *)ctx->partials;
       args.tiles_m = args.m / 256;
       args.tiles_n = args.n / 256;
       hipLaunchKernelGGL((gemm_nt_dma4_kernel<KIND, OUT_F32, 256, 256, 128, 2, 2, true>),
@@ -1143,10 +1163,10 @@ int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
       return launch_status("gemm_fold_kernel");
     }
   }
-  if (args.kbytes % 128 != 0) return launch_wave8<KIND, OUT, 64>(st, args);
-  long ns = 0;
-  const int tile = pick_tile(args.m, args.n, args.kbytes, OUT == OUT_SWIGLU, cus, &ns);
-  return tile < 0 ? launch_wave8<KIND, OUT, 128>(st, args) : launch_tile<KIND, OUT>(st, args, tile);
+  if (r.kernel == ROUTE_WAVE8)
+    return args.kbytes % 128 == 0 ? launch_wave8<KIND, OUT, 128>(st, args, r.bm)
+                                  : launch_wave8<KIND, OUT, 64>(st, args, r.bm);
+  return launch_tile4<KIND, OUT>(st, args, r.bm, r.bn);
 }
 
 int relayout_rhs(wafer_hip_context *ctx, const void *rhs, uint32_t k, uint32_t n, int esize,
@@ -1199,6 +1219,16 @@ int check_shape(uint32_t m, uint32_t k, uint32_t n, int esize, const char *what)
 
 using namespace wafer;
 
+// For the dispatch tests, host only: the route of a product on a chip of `cus`
+// CUs (kind and out as in gemm_common.h) as kernel, bm, bn, ksplit.
+extern "C" void wafer_internal_gemm_route(int kind, int out, int m, int n, int kbytes, int cus, int *route) {
+  const GemmRoute r = gemm_route(kind, out, m, n, kbytes, cus);
+  route[0] = r.kernel;
+  route[1] = r.bm;
+  route[2] = r.bn;
+  route[3] = r.ksplit;
+}
+
 extern "C" int wafer_hip_gemm_mfma(wafer_hip_context *ctx, const void *lhs, const void *rhs,
                                    void *dst, uint32_t m, uint32_t k, uint32_t n,
                                    uint32_t in_format, uint32_t out_format,
@@ -1215,7 +1245,6 @@ extern "C" int wafer_hip_gemm_mfma(wafer_hip_context *ctx, const void *lhs, cons
   const uint8_t *bt = (const uint8_t *)rhs;
   if (rhs_orientation == WAFER_GEMM_NORMAL) WAFER_TRY(relayout_rhs(ctx, rhs, k, n, 2, &bt));
   GemmArgs args{(const uint8_t *)lhs, bt, dst, nullptr, nullptr, (int)m, (int)n, (int)(k * 2), 0, 0};
-  WAFER_TRY(prepare_split(ctx, args));
   const bool f32 = out_format == WAFER_FMT_F32;
   if (in_format == WAFER_FMT_BF16)
     return f32 ? launch_gemm<KIND_BF16, OUT_F32>(ctx, args)
@@ -1238,7 +1267,6 @@ extern "C" int wafer_hip_gemm_mfma_residual(wafer_hip_context *ctx, const void *
   if (rhs_orientation == WAFER_GEMM_NORMAL) WAFER_TRY(relayout_rhs(ctx, rhs, k, n, 2, &bt));
   GemmArgs args{(const uint8_t *)lhs, bt, dst, nullptr, nullptr, (int)m, (int)n, (int)(k * 2), 0, 0,
                 (const uint16_t *)residual};
-  WAFER_TRY(prepare_split(ctx, args));
   return in_format == WAFER_FMT_BF16 ? launch_gemm<KIND_BF16, OUT_NARROW_RES>(ctx, args)
                                      : launch_gemm<KIND_F16, OUT_NARROW_RES>(ctx, args);
 }
