@@ -93,7 +93,11 @@ __device__ inline uint16_t swiglu_pair(float a, float b) {
 // XCD-aware tile order: workgroup ids are dealt round-robin over the 8
 // XCDs; the ids one XCD receives cover a 4 x 8 block of output tiles when the
 // grid is whole rounds of 256 tiles, else (tile rows divisible by 4, tile
-// columns by 8) the XCD's own column strip walked in 4-row groups.
+// columns by 8) the XCD's own column strip walked in 4-row groups.  RUNS: the
+// order of the other grids on the 4-wave kernel; the 8-wave kernel walks them
+// row by row (64-byte stages, K 1056: 1152 x 4096 23 us against 26 in runs, 1152 x
+// 14336 56 / 66; 128-byte stages equal).
+template <bool RUNS>
 __device__ inline void tile_coords(const GemmArgs &args, int bid, int &tm, int &tn) {
   const int tiles_m = args.tiles_m, tiles_n = args.tiles_n;
   const int total = tiles_m * tiles_n;
@@ -114,6 +118,9 @@ __device__ inline void tile_coords(const GemmArgs &args, int bid, int &tm, int &
     const int grp = j / per_group, w = j % per_group;
     tm = grp * 4 + w % 4;
     tn = xcd * sw + w / 4;
+  } else if constexpr (!RUNS) {
+    tm = bid / tiles_n;
+    tn = bid % tiles_n;
   } else {
     // any other grid: XCD x takes a contiguous run of the tiles, walked in
     // groups of up to 8 tile rows, column by column within a group, so that
@@ -370,7 +377,7 @@ gemm_nt_kernel(GemmArgs args) {
   };
 
   int tm, tn;
-  tile_coords(args, blockIdx.x, tm, tn);
+  tile_coords<false>(args, blockIdx.x, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -704,7 +711,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int tiles = args.tiles_m * args.tiles_n;
   const int split = SPLIT ? (int)blockIdx.x / tiles : 0;
   int tm, tn;
-  tile_coords(args, (int)blockIdx.x - split * tiles, tm, tn);
+  tile_coords<true>(args, (int)blockIdx.x - split * tiles, tm, tn);
   // SHIFT: the last tile row / column starts early enough to end at m / n,
   // and stores only what the tile before it does not
   const int row_lo = tm * BM, col_lo = tn * BN;
