@@ -57,3 +57,16 @@ def test_swiglu_takes_the_tile_it_was_priced_on(lib, m, features, k, route):
     tiles take the 8-wave kernel over rows of 3 or 5 times a power of two bytes."""
     for kind in (K_BF16, K_F16):
         assert gemm_route(lib, m, 2 * features, k, OUT_SWIGLU, kind) == route
+
+
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (777, 4096, 2048, TILE4), (777, 4096, 4096, WAVE8), (200, 14336, 4096, WAVE8), (600, 4096, 4096, WAVE8),
+    (1024, 4096, 4096, TILE4), (896, 4096, 12288, WAVE8), (900, 4096, 14336, WAVE8)])
+@pytest.mark.parametrize("out", [OUT_F32, OUT_NARROW, OUT_RES])
+def test_ragged_128_tiles_take_the_8_wave_kernel(lib, m, n, k, kernel, out):
+    """128x128 tiles over 16-bit operands from K 4096 on: the 8-wave kernel where
+    they do not divide the output, and from K 12288 on everywhere."""
+    for kind in (K_BF16, K_F16):
+        assert gemm_route(lib, m, n, k, out, kind) == (kernel, 128, 128, 1)
+    if kernel == WAVE8 and k < 12288:
+        assert gemm_route(lib, m, n, k, OUT_I8, K_I8)[0] == TILE4

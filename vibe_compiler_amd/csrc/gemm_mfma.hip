@@ -1084,11 +1084,14 @@ GemmRoute gemm_route(int kind, int out, int m, int n, int kbytes, int cus) {
     // 12288 202 / 335).
     const int odd = kbytes / (kbytes & -kbytes);
     if (r.bm == 256 && r.bn == 256 && (odd == 3 || odd == 5)) return wave8;
-  } else if (r.bm == 128 && r.bn == 128 && kbytes >= 24576) {
-    // past K 12288 the 8-wave kernel serves 128x128 tiles (777 x 4096, K 14336:
-    // 127 us against 145; K 11008: 101 against 102; 900 x 4096, K 8192: 83
-    // against 72)
-    return wave8;
+  } else if (r.bm == 128 && r.bn == 128) {
+    // 128x128 tiles, 4-wave / 8-wave us: 16-bit rows or columns that they do not
+    // divide go to the 8-wave kernel from K 4096 on (777 x 4096: K 2048 19.9 /
+    // 21.0, 4096 44.6 / 37.1, 8192 88 / 71, 12288 148 / 113; 200 x 14336, K 4096
+    // 46 / 42; 900 x 4096 39.8 / 40.0), whole grids past K 12288 (1152 x 4096: K
+    // 8192 124 / 129, 12288 268 / 201, 14336 270 / 241).
+    const bool whole = m % 128 == 0 && n % 128 == 0;
+    if (kbytes >= 24576 || (!i8 && !whole && kbytes >= 8192)) return wave8;
   }
   return r;
 }
