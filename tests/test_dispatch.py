@@ -18,10 +18,10 @@ def lib():
     return backend.load()
 
 
-def gemm_route(lib, m, n, k, out=OUT_NARROW, kind=K_BF16, cus=256):
+def gemm_route(lib, m, n, k, out=OUT_NARROW, kind=K_BF16, acc=False, cus=256):
     """(kernel, tile rows, tile columns, splits) of m x n outputs over k elements; n counts a SwiGLU's two products."""
     r = (ctypes.c_int * 4)()
-    lib.wafer_internal_gemm_route(kind, out, m, n, k * (1 if kind == K_I8 else 2), cus, r)
+    lib.wafer_internal_gemm_route(kind, out, m, n, k * (1 if kind == K_I8 else 2), cus, int(acc), r)
     return tuple(r)
 
 
@@ -70,3 +70,20 @@ def test_ragged_128_tiles_take_the_8_wave_kernel(lib, m, n, k, kernel, out):
         assert gemm_route(lib, m, n, k, out, kind) == (kernel, 128, 128, 1)
     if kernel == WAVE8 and k < 12288:
         assert gemm_route(lib, m, n, k, OUT_I8, K_I8)[0] == TILE4
+
+
+@pytest.mark.parametrize("m,n,plain,acc", [
+    (300, 4096, (TILE4, 128, 64), (TILE4, 128, 64)), (1024, 4096, (TILE4, 128, 128), (TILE4, 128, 128)),
+    (512, 4096, (TILE4, 128, 64), (WAVE8, 128, 128)), (777, 4096, (TILE4, 128, 128), (WAVE8, 128, 128)),
+    (4096, 1000, (TILE4, 128, 128), (WAVE8, 128, 128)), (1152, 4096, (TILE4, 128, 192), (WAVE8, 128, 128)),
+    (256, 4096, (TILE4, 64, 64), (TILE4, 64, 64)), (777, 6144, (TILE4, 128, 192), (TILE4, 128, 192)), (4096, 4096, (WAVE8, 256, 256), (WAVE8, 256, 256))])
+def test_int8_accumulators_keep_the_faster_kernel(lib, m, n, plain, acc):
+    """An int8 product whose accumulators are asked for stores them element by
+    element: shifted tiles, and 128x64 where whole 128x128 ones serve, are slower so."""
+    assert gemm_route(lib, m, n, 4096, OUT_I8, K_I8)[:3] == plain
+    assert gemm_route(lib, m, n, 4096, OUT_I8, K_I8, acc=True)[:3] == acc
+
+
+def test_int8_128_tiles_over_a_short_k(lib):
+    for k, kernel in ((512, WAVE8), (1024, WAVE8), (1152, TILE4), (4096, TILE4)):
+        assert gemm_route(lib, 1024, 4096, k, OUT_I8, K_I8)[:3] == (kernel, 128, 128)

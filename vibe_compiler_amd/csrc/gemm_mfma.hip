@@ -1051,11 +1051,12 @@ int plan_split(int m, int n, int kbytes, int cus) {
 }
 
 // Which kernel serves a product of m x n (n counts both products of a
-// SwiGLU), and on which tile; what is priced here is what is launched.
+// SwiGLU), and on which tile; what is priced here is what is launched.  acc: the
+// int8 accumulators are asked for too, which go out element by element.
 enum { ROUTE_STREAM = 0, ROUTE_TILE4 = 1, ROUTE_WAVE8 = 2, ROUTE_SPLIT = 3 };
 struct GemmRoute { int kernel, bm, bn, ksplit; };
 
-GemmRoute gemm_route(int kind, int out, int m, int n, int kbytes, int cus) {
+GemmRoute gemm_route(int kind, int out, int m, int n, int kbytes, int cus, bool acc = false) {
   const bool swiglu = out == OUT_SWIGLU, i8 = kind == KIND_I8;
   if (gemm_is_skinny(m, swiglu ? n / 2 : n, cus)) return {ROUTE_STREAM, 0, 0, 1};
   if (!i8 && !swiglu) {
@@ -1074,6 +1075,15 @@ GemmRoute gemm_route(int kind, int out, int m, int n, int kbytes, int cus) {
     if (m % 256 == 0 && n % 256 == 0) return wave8;
     r.bm = r.bn = 128;
   }
+  const bool whole = m % 128 == 0 && n % 128 == 0;
+  if (acc) {
+    // the 4-wave kernel only where it was the faster one (300 x 4096 and 1024 x
+    // 4096, K 4096, 4-wave / 8-wave us: 20.2 / 23.8, 25.3 / 26.1): not for shifted
+    // 128x128 tiles (777 x 4096 30.5 / 27.4), shifted columns of 128x192 (1152 x
+    // 4096 42.7 / 39.2), or 128x64 where whole 128x128 ones serve (512 x 4096 21.1 /
+    // 19.6; 64x64 stay: 256 x 4096 14.7 / 18.5)
+    if (r.bn == 192 ? n % 192 != 0 : r.bm == 128 && r.bn == 128 ? !whole : r.bm == 128 && whole) return wave8;
+  }
   if (swiglu) {
     // 256x256 tiles over a K row of 3 or 5 times a power of two bytes: the
     // 4-wave kernel's time jumps there (300 x 2 * 11008, 4-wave / 8-wave us: K
@@ -1089,9 +1099,9 @@ GemmRoute gemm_route(int kind, int out, int m, int n, int kbytes, int cus) {
     // divide go to the 8-wave kernel from K 4096 on (777 x 4096: K 2048 19.9 /
     // 21.0, 4096 44.6 / 37.1, 8192 88 / 71, 12288 148 / 113; 200 x 14336, K 4096
     // 46 / 42; 900 x 4096 39.8 / 40.0), whole grids past K 12288 (1152 x 4096: K
-    // 8192 124 / 129, 12288 268 / 201, 14336 270 / 241).
-    const bool whole = m % 128 == 0 && n % 128 == 0;
-    if (kbytes >= 24576 || (!i8 && !whole && kbytes >= 8192)) return wave8;
+    // 8192 124 / 129, 12288 268 / 201, 14336 270 / 241).  int8 over a short K too
+    // (1024 x 4096, K 1024 11.3 / 9.9; K 4096 25.3 / 25.9, 2048 rows 39.2 / 43.3).
+    if (kbytes >= 24576 || (i8 ? whole && kbytes <= 1024 : !whole && kbytes >= 8192)) return wave8;
   }
   return r;
 }
@@ -1153,7 +1163,7 @@ template <int KIND, int OUT>
 int launch_gemm(wafer_hip_context *ctx, GemmArgs args) {
   const hipStream_t st = ctx->stream;
   const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-  const GemmRoute r = gemm_route(KIND, OUT, args.m, args.n, args.kbytes, cus);
+  const GemmRoute r = gemm_route(KIND, OUT, args.m, args.n, args.kbytes, cus, args.acc_out != nullptr);
   if (r.kernel == ROUTE_STREAM) return launch_gemm_skinny<KIND, OUT>(st, args, cus);
   if constexpr (KIND != KIND_I8 && OUT != OUT_SWIGLU) {
     if (r.kernel == ROUTE_SPLIT) {
@@ -1230,9 +1240,10 @@ int check_shape(uint32_t m, uint32_t k, uint32_t n, int esize, const char *what)
 using namespace wafer;
 
 // For the dispatch tests, host only: the route of a product on a chip of `cus`
-// CUs (kind and out as in gemm_common.h) as kernel, bm, bn, ksplit.
-extern "C" void wafer_internal_gemm_route(int kind, int out, int m, int n, int kbytes, int cus, int *route) {
-  const GemmRoute r = gemm_route(kind, out, m, n, kbytes, cus);
+// CUs (kind and out as in gemm_common.h; acc: with int8 accumulators) as kernel,
+// bm, bn, ksplit.
+extern "C" void wafer_internal_gemm_route(int kind, int out, int m, int n, int kbytes, int cus, int acc, int *route) {
+  const GemmRoute r = gemm_route(kind, out, m, n, kbytes, cus, acc != 0);
   route[0] = r.kernel;
   route[1] = r.bm;
   route[2] = r.bn;
