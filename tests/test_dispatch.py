@@ -87,3 +87,16 @@ def test_int8_accumulators_keep_the_faster_kernel(lib, m, n, plain, acc):
 def test_int8_128_tiles_over_a_short_k(lib):
     for k, kernel in ((512, WAVE8), (1024, WAVE8), (1152, TILE4), (4096, TILE4)):
         assert gemm_route(lib, 1024, 4096, k, OUT_I8, K_I8)[:3] == (kernel, 128, 128)
+
+
+@pytest.mark.parametrize("fmt,group_size,rows,keys,chunks,group,fused", [
+    (BF16, 1, 1024, 17, 16, 1, 0), (BF16, 1, 512, 300, 16, 1, 1), (F16, 1, 512, 2048, 16, 1, 0),
+    (BF16, 4, 256, 1, 16, 1, 0), (F16, 1, 32, 4095, 16, 0, 1), (BF16, 8, 256, 1, 16, 0, 0), (BF16, 8, 256, 17, 1, 0, 1),
+    (BF16, 8, 128, 17, 16, 0, 1), (BF16, 8, 128, 17, 32, 0, 0), (BF16, 8, 64, 8192, 16, 0, 1),
+    (BF16, 8, 64, 8193, 16, 0, 0), (F16, 4, 256, 300, 16, 0, 1), (F16, 1, 1, (1 << 32) - 1, 16, 0, 0)])
+def test_decode_append_rule(lib, fmt, group_size, rows, keys, chunks, group, fused):
+    """A decode step's new rows are written by the decode kernel only where that
+    beats a copy kernel before it: not over large caches or many workgroups."""
+    u32 = ctypes.c_uint32
+    assert lib.wafer_internal_append_in_kernel(u32(fmt), u32(group_size), u32(rows), u32(keys), u32(chunks), group,
+                                               u32(256)) == fused

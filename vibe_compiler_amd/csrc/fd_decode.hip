@@ -443,6 +443,20 @@ bool takes_group(const wafer_hip_context *ctx, uint32_t format, uint32_t G, uint
   return G <= gmax && chunks <= (uint32_t)WG_WAVES && (uint64_t)batch * kv_heads * 4 >= (uint64_t)cus * 3;
 }
 
+// Whether the decode kernels write a step's new rows themselves, which saves
+// the copy kernel's launch (2.0 us).  The row selects cost 10 to 45 registers
+// and show where the caches are past 256 MiB or the workgroups many (copy
+// kernel / in the decode kernel, us: 32 x 32 heads, 17 keys 20.0 / 22.3, 1000
+// keys 86 / 89; 16 x 32 heads, 2048 keys 86 / 92; 64 over 8 heads, 32 x 8192 keys
+// 197 / 203, 32 x 1 56.4 / 59.0; but 16 x 32 heads, 300 keys 20.9 / 20.2, 32 heads,
+// 8192 keys 32.1 / 26.5).  BF16 groups of 4 on one workgroup would spill.
+bool appends_in_kernel(uint32_t format, uint64_t G, uint64_t rows, uint64_t keys, uint64_t chunks, bool group,
+                       uint64_t cus) {
+  if (rows * keys > 1u << 19) return false;
+  if (group) return rows <= 2 * cus && !(format == WAFER_FMT_BF16 && G == 4);
+  return G * rows * chunks <= 64 * cus;
+}
+
 // Shared by the entries: validation, then the group path (no workspace) or
 // the chunk grid plus fold, whose states go to the no-allocation scratch or to
 // the context's workspace (grown on demand).  k_new / v_new: row kv_len - 1 of
@@ -500,7 +514,7 @@ int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k
       switch (G) {
       case 1: FD_GROUP(__bf16, 1); break;
       case 2: FD_GROUP(__bf16, 2); break;
-      default: FD_GROUP1(__bf16, 4, false); break;  // (with the append it would spill)
+      default: FD_GROUP1(__bf16, 4, false); break;  // (appends_in_kernel)
       }
     } else {
       switch (G) {
@@ -623,6 +637,12 @@ int noalloc_scratch_lookup(int device) {
 
 using namespace wafer;
 
+// For the dispatch tests, host only.
+extern "C" int wafer_internal_append_in_kernel(uint32_t format, uint32_t G, uint32_t rows, uint32_t keys,
+                                               uint32_t chunks, int group, uint32_t cus) {
+  return appends_in_kernel(format, G, rows, keys, chunks, group != 0, cus);
+}
+
 extern "C" int wafer_hip_attention_decode(wafer_hip_context *ctx, uint32_t format,
                                           const void *q, const void *k_cache,
                                           const void *v_cache, void *o, uint32_t batch,
@@ -676,8 +696,11 @@ extern "C" int wafer_hip_attention_decode_append(wafer_hip_context *ctx, uint32_
   const bool vec = head_dim % 8 == 0 &&
                    (((uintptr_t)k_new | (uintptr_t)v_new | (uintptr_t)k_cache | (uintptr_t)v_cache) & 15) == 0;
   // one token at head_dim 128: the decode kernels write the new rows
-  // themselves (a launch of 1.7 us and its gap less)
-  if (fd && vec && !(q_heads / kv_heads == 4 && takes_group(ctx, format, 4, chunks, batch, kv_heads)))
+  // themselves where that is the faster way
+  if (fd && vec &&
+      appends_in_kernel(format, q_heads / kv_heads, (uint64_t)batch * kv_heads, (uint64_t)past_len + 1, chunks,
+                        takes_group(ctx, format, q_heads / kv_heads, chunks, batch, kv_heads),
+                        ctx->cu_count > 0 ? ctx->cu_count : 256))
     return decode(ctx, format, q, k_cache, v_cache, o, batch, q_heads, kv_heads, past_len + 1, kv_capacity, head_dim,
                   scale, chunks, false, k_new, v_new);
   const int piece_elems = vec ? 8 : 1;
