@@ -195,7 +195,11 @@ def test_decode_append_rejects_overflow_without_writing(hip):
 @pytest.mark.parametrize("fmt", [2, 3], ids=["f16", "bf16"])
 @pytest.mark.parametrize("Bn,Hq,Hkv,L,chunks", [
     (1, 8, 8, 1, 16), (1, 8, 4, 17, 1), (1, 4, 4, 129, 1), (1, 4, 1, 3231, 16), (2, 8, 1, 1000, 3), (1, 2, 2, 8191, 4),
-    (24, 16, 8, 260, 16), (24, 32, 8, 130, 16), (3, 8, 8, 700, 20)])
+    (24, 16, 8, 260, 16), (24, 32, 8, 130, 16), (3, 8, 8, 700, 20),
+    # one to five states to fold; the append on one workgroup per head, before
+    # it (many workgroups), and on the chunk grid of groups of 8 either way
+    (1, 8, 4, 40, 2), (1, 4, 4, 40, 3), (2, 8, 1, 60, 4), (1, 8, 4, 60, 5), (24, 8, 8, 100, 16), (130, 8, 8, 40, 16),
+    (16, 64, 8, 40, 16), (32, 64, 8, 40, 16)])
 def test_split_chunks_and_fused_append(hip, fmt, Bn, Hq, Hkv, L, chunks):
     """The chunk grid with chunks split over workgroups (one part of 16 keys to
     several, parts past the end empty) and the one-workgroup path, against

@@ -365,11 +365,12 @@ __global__ __launch_bounds__(256) void fd_chunk_d128(
 // for 16 states.  P groups of 128 threads each fold a run of the states, the
 // loads of 8 states out together, and the runs' states fold left to right
 // through LDS.  A decode step over 32 x 4095 keys (append, chunks, fold):
-// 20.7 -> 15.7 us.
+// 20.7 -> 15.7 us.  Up to four states one group folds alone (2048 heads of 4
+// states, with the chunks: two groups 21.5, one 19.7 us).
 template <typename T, int P>
 __global__ __launch_bounds__(128 * P) void fd_fold_d128(const ChunkState *__restrict__ part,
                                                         uint16_t *__restrict__ O, int states) {
-  constexpr int NB = 8;
+  constexpr int NB = P == 1 ? 4 : 8;
   __shared__ float sA[P][D], sM[P], sL[P];
   const int bh = blockIdx.x, d = threadIdx.x % D, run = threadIdx.x / D;
   const ChunkState *ps = part + (size_t)bh * states;
@@ -580,10 +581,12 @@ int decode(wafer_hip_context *ctx, uint32_t format, const void *q, const void *k
                      nstates)
   if (format == WAFER_FMT_BF16) {
     if (nstates > 16) FD_FOLD(__bf16, 8);
-    else FD_FOLD(__bf16, 2);
+    else if (nstates > 4) FD_FOLD(__bf16, 2);
+    else FD_FOLD(__bf16, 1);
   } else {
     if (nstates > 16) FD_FOLD(_Float16, 8);
-    else FD_FOLD(_Float16, 2);
+    else if (nstates > 4) FD_FOLD(_Float16, 2);
+    else FD_FOLD(_Float16, 1);
   }
 #undef FD_FOLD
   return launch_status("fd_fold_d128");
