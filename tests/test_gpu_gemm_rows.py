@@ -1,8 +1,8 @@
 """GPU tests of the MFMA GEMMs by row count: the weight-streaming kernel of few
 rows, at the edges of its 16-row tiles and of its column tiles, and with K
 that is not a whole 128-byte unit or leaves some of a workgroup's waves
-without one; and the 4-wave tile kernel where its tiles do not divide the
-output.
+without one; and every tile of the 4-wave and 8-wave kernels and the K split, each
+checked to be the one the dispatch takes.
 
 Against float64 on the same inputs: an f32 sum of K products in any order is
 within K 2^-24 sum |a| |b| of the exact one.  A 16-bit output adds half an ulp:
@@ -46,17 +46,81 @@ def _check(got, a, b, half_ulp):
 
 ROWS = [(1, 128, 4096, 3), (15, 130, 96, 2), (16, 16, 32, 3), (17, 4096, 160, 3), (31, 33, 8192, 2), (32, 8192, 96, 3),
         (33, 1000, 544, 2), (48, 10272, 64, 3), (63, 20, 2080, 3), (64, 12288, 128, 2), (64, 640, 1024, 3)]
-# few outputs of more rows (64 x 32 tiles, SwiGLU 64 x 64), and tiles of the
-# 4-wave kernel whose last row / column of tiles is shifted back to the edge:
-# 64x64, 64x128, 128x64, 128x128, 128x192 and 256x256, with n of every alignment
+# few outputs of more rows (64 x 32 tiles, SwiGLU 64 x 64), and more of them with
+# n of every alignment
 TILES = [(200, 4100, 128, 3), (65, 64, 128, 3), (127, 72, 256, 2), (100, 16400, 128, 3), (129, 130, 192, 2), (300, 4100, 128, 3),
          (300, 6145, 256, 2), (1000, 6148, 128, 3), (300, 28648, 64, 2), (300, 28656, 128, 3), (130, 60, 256, 3),
          (1000, 500, 96, 2), (120, 4096, 2080, 3)]
 
 
+# every kernel and tile of more rows, by its route (kernel, tile rows, tile
+# columns, splits; test_dispatch.py): whole grids, and grids whose last row,
+# column or both the tile does not divide, BF16 and F16 in turn
+TILE4, WAVE8, SPLIT = 1, 2, 3
+ROUTES = [
+    (64, 64, TILE4, (65, 4100, 64), (65, 4160, 192), (128, 4100, 64), (200, 4096, 4096)),
+    (64, 128, TILE4, (65, 8200, 128), (320, 6144, 64), (65, 11008, 64), (192, 8200, 64)),
+    (128, 64, TILE4, (129, 6148, 64), (256, 4160, 64), (129, 6144, 128), (128, 8200, 64)),
+    (128, 128, TILE4, (200, 8200, 64), (384, 6144, 192), (129, 11008, 64), (256, 8200, 64), (700, 4100, 2048)),
+    (128, 192, TILE4, (257, 11008, 64), (384, 12288, 64), (257, 12288, 128), (512, 8200, 64), (700, 6148, 4096)),
+    (256, 256, TILE4, (16448, 320, 64), (768, 8192, 64), (1024, 6148, 128), (1000, 6145, 64)),
+    # 8 waves: long K, 64-byte K stages, and products narrower than every tile
+    (128, 128, WAVE8, (384, 6144, 12288), (129, 11008, 4096), (256, 8200, 4096), (700, 4100, 14336), (16448, 32, 64),
+     (65, 4100, 32), (384, 1536, 96), (129, 3072, 4128), (128, 4100, 32), (1024, 4096, 96)),
+    (256, 256, WAVE8, (1024, 12288, 32), (1024, 12288, 96)),
+    (256, 256, SPLIT, (768, 1536, 10240), (512, 4096, 14336), (768, 3072, 8192)),
+]
+ROUTED = [(*s, 3 if (i + s[0]) % 2 else 2, (kernel, bm, bn)) for bm, bn, kernel, *shapes in ROUTES
+          for i, s in enumerate(shapes)]
+# the same of SwiGLU products (n features)
+SWIGLU_ROUTES = [
+    (64, 128, TILE4, (400, 2080, 64), (320, 3072, 64), (65, 5504, 128)),
+    (128, 64, TILE4, (256, 2080, 64), (129, 3072, 64)),
+    (128, 128, TILE4, (500, 2080, 64), (384, 3072, 64), (129, 5504, 64), (512, 2080, 128), (129, 5504, 12352)),
+    (128, 192, TILE4, (257, 5504, 64), (384, 6144, 64), (257, 6144, 128), (384, 5504, 64)),
+    (256, 224, TILE4, (512, 7168, 64), (512, 7168, 192)),
+    (256, 256, TILE4, (768, 4096, 64), (1536, 2080, 64), (777, 5520, 128)),
+    (256, 256, WAVE8, (768, 4096, 192), (1536, 2080, 192), (777, 5520, 320), (768, 768, 32), (65, 5504, 96),
+     (256, 2080, 32)),
+]
+SWIGLU_ROUTED = [(*s, 3 if (i + s[0]) % 2 else 2, (kernel, bm, bn)) for bm, bn, kernel, *shapes in SWIGLU_ROUTES
+                 for i, s in enumerate(shapes)]
+
+
+def _route(B, m, n, k, swiglu=False):
+    import ctypes
+
+    r = (ctypes.c_int * 4)()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    B.load().wafer_internal_gemm_route(0, 3 if swiglu else 1, m, n, 2 * k, cus, 0, r)
+    return tuple(r)[:3]
+
+
 @pytest.mark.parametrize("m,n,k,fmt", ROWS + TILES)
 def test_gemm_rows_vs_float64(hip, B, m, n, k, fmt):
     print("[gemm rows]", m, n, k, fmt, flush=True)
+    _rows(hip, B, m, n, k, fmt)
+
+
+@pytest.mark.parametrize("m,n,k,fmt,route", ROUTED)
+def test_gemm_routes_vs_float64(hip, B, m, n, k, fmt, route):
+    print("[gemm route]", m, n, k, fmt, route, flush=True)
+    assert _route(B, m, n, k) == route
+    split = route[0] == SPLIT
+    _rows(hip, B, m, n, k, fmt, swiglu=False, shifts=(0,) if split else (0, 1))
+
+
+@pytest.mark.parametrize("m,n,k,fmt,route", SWIGLU_ROUTED)
+def test_swiglu_routes_vs_plain(hip, B, m, n, k, fmt, route):
+    print("[swiglu route]", m, n, k, fmt, route, flush=True)
+    assert _route(B, m, 2 * n, k, swiglu=True) == route
+    dt = torch.bfloat16 if fmt == B.BF16 else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(m * 7 + n * 3 + k)
+    _swiglu(hip, B, (torch.randn(m, k, generator=g, device="cuda")).to(dt),
+            (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(dt), g, m, n, k, fmt)
+
+
+def _rows(hip, B, m, n, k, fmt, swiglu=True, shifts=(0, 1)):
     dt, half_ulp = (torch.bfloat16, 2.0 ** -8) if fmt == B.BF16 else (torch.float16, 2.0 ** -11)
     g = torch.Generator(device="cuda").manual_seed(m * 7 + n * 3 + k)
     a = torch.randn(m, k, generator=g, device="cuda").to(dt)
@@ -66,7 +130,7 @@ def test_gemm_rows_vs_float64(hip, B, m, n, k, fmt):
     _check(out[:m * n].view(m, n), a, b, 0.0)
     assert torch.all(out[m * n:] == 7.5)
     # an output that no vector store is aligned for
-    for shift in (0, 1):
+    for shift in shifts:
         outn = torch.full((m * n + 512,), 7.5, dtype=dt, device="cuda")
         view = outn[shift:shift + m * n]
         hip.gemm_mfma(a, b, view, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
@@ -78,20 +142,30 @@ def test_gemm_rows_vs_float64(hip, B, m, n, k, fmt):
     hip.elementwise("Add", fmt, view.clone().view(m, n), ref, r)
     hip.gemm_mfma_residual(a, b, r, r, m, k, n, in_fmt=fmt, rhs_t=True)
     assert torch.equal(r.view(torch.int16), ref.view(torch.int16))
-    if n % 16 == 0:  # SwiGLU of n features
-        wu = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(dt)
-        gate, up, ref, got = (torch.empty(m, n, dtype=dt, device="cuda") for _ in range(4))
-        hip.gemm_mfma(a, b, gate, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
-        hip.gemm_mfma(a, wu, up, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
-        hip.silu_mul(gate, up, ref, fmt=fmt)
-        packed = torch.empty(2 * n, k, dtype=dt, device="cuda")
-        hip.interleave_gate_up(b, wu, packed)
-        hip.gemm_mfma_swiglu(a, packed, got, m, k, n, in_fmt=fmt)
-        assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+    if swiglu and n % 16 == 0:
+        _swiglu(hip, B, a, b, g, m, n, k, fmt)
+
+
+def _swiglu(hip, B, a, b, g, m, n, k, fmt):
+    """The SwiGLU of n features (gate weights b) is the two narrowed products and the region, bit for bit."""
+    wu = (torch.randn(n, k, generator=g, device="cuda") * k ** -0.5).to(a.dtype)
+    gate, up, ref, got = (torch.empty(m, n, dtype=a.dtype, device="cuda") for _ in range(4))
+    hip.gemm_mfma(a, b, gate, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
+    hip.gemm_mfma(a, wu, up, m, k, n, in_fmt=fmt, out_fmt=fmt, rhs_t=True)
+    hip.silu_mul(gate, up, ref, fmt=fmt)
+    packed = torch.empty(2 * n, k, dtype=a.dtype, device="cuda")
+    hip.interleave_gate_up(b, wu, packed)
+    hip.gemm_mfma_swiglu(a, packed, got, m, k, n, in_fmt=fmt)
+    assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 100, 64), (16, 4096, 1024), (33, 1001, 4160), (64, 12288, 192),
-                                   (65, 100, 256), (300, 1000, 1024), (301, 4103, 128), (777, 6151, 128)])
+                                   (65, 100, 256), (300, 1000, 1024), (301, 4103, 128), (777, 6151, 128),
+                                   # 4-wave tiles 64x64, 64x128, 128x64, 128x128, 128x192 and the 8-wave kernel
+                                   # (64-byte stages, a short K, whole 256x256)
+                                   (65, 4100, 128), (192, 8200, 128), (129, 6148, 128), (384, 6144, 2048),
+                                   (200, 8200, 128), (512, 8200, 128), (257, 12288, 128), (300, 4103, 4160),
+                                   (1024, 4096, 192), (384, 6144, 128), (1024, 12288, 64), (1024, 12288, 128)])
 @pytest.mark.parametrize("rt", [False, True])
 def test_gemm_i8_rows_bit_exact(hip, B, m, n, k, rt):
     print("[gemm i8 rows]", m, n, k, rt, flush=True)

@@ -107,12 +107,23 @@ def test_i8_gemm_kn_graph_replay(hip):
                          lambda: hip.gemm_i8(a2, b, sc, y2, m, k, n))
 
 
+def splits(B, m, n, k):
+    """How many ways the dispatch splits K of a 16-bit product (0: not at all)."""
+    import ctypes
+
+    r = (ctypes.c_int * 4)()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    B.load().wafer_internal_gemm_route(0, 0, m, n, 2 * k, cus, 0, r)
+    return r[3] if r[0] == 3 else 0
+
+
 def test_mfma_gemm_split_k_graph_replay(hip, B):
     """bf16 MFMA GEMM on the split-K schedule: f32 partial tiles in the
     context's area (grown by the eager call), then the fold launch."""
     say("graph replay: mfma gemm split-k")
     gen = torch.Generator(device="cuda").manual_seed(14)
-    m, k, n = 256, 8192, 1024
+    m, k, n = 768, 10240, 1536
+    assert splits(B, m, n, k)
     a, a2 = rnd((m, k), gen), rnd((m, k), gen)
     bt = rnd((n, k), gen)
     y, y2 = (torch.empty((m, n), dtype=torch.float32, device="cuda") for _ in range(2))
@@ -144,8 +155,9 @@ def test_graph_survives_workspace_growth(B):
     say("graph replay across workspace growth")
     hip = B.Context(0)
     gen = torch.Generator(device="cuda").manual_seed(16)
-    k, n = 8192, 1024
-    small_m, big_m = 256, 1024   # 4 and 16 MiB of f32 partials (4 splits)
+    k, n = 14336, 1536
+    small_m, big_m = 768, 2048   # 18 and 48 MiB of f32 partials (4 splits)
+    assert splits(B, small_m, n, k) == splits(B, big_m, n, k) == 4
     a = rnd((small_m, k), gen)
     bt = rnd((n, k), gen)
     y = torch.empty((small_m, n), dtype=torch.float32, device="cuda")
@@ -166,7 +178,7 @@ def test_graph_survives_workspace_growth(B):
     y_big = torch.empty((big_m, n), dtype=torch.float32, device="cuda")
     hip.gemm_mfma(a_big, bt, y_big, big_m, k, n, in_fmt=B.BF16, out_fmt=B.F32, rhs_t=True)
     torch.cuda.synchronize()
-    canary = torch.full((8 << 20,), 3.0, dtype=torch.float32, device="cuda")  # 32 MiB allocated after the growth
+    canary = torch.full((16 << 20,), 3.0, dtype=torch.float32, device="cuda")  # 64 MiB allocated after the growth
     for r in range(3):
         y.zero_()
         torch.cuda.synchronize()
