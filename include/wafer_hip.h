@@ -141,7 +141,10 @@ int wafer_hip_gemm(wafer_hip_context *ctx, const void *lhs, const void *rhs,
  * and n multiples of 256) may split K over 4 workgroups with f32 partials in a
  * context-owned area (4 * m * n * 4 bytes, grown on first use; growing is
  * refused on a capturing stream, so a caller that captures runs the shape
- * once eagerly first).  Results repeat bit for bit for a given shape. */
+ * once eagerly first).  Results repeat bit for bit for a given shape.  The
+ * order of a sum depends on the kernel, which m, n, k and the CU count choose
+ * (few rows or few outputs: K in 128-byte units over four waves; a K split; else
+ * k order), so a row's bits may differ with the rows that come with it. */
 int wafer_hip_gemm_mfma(wafer_hip_context *ctx, const void *lhs,
                         const void *rhs, void *dst, uint32_t m, uint32_t k,
                         uint32_t n, uint32_t in_format, uint32_t out_format,
@@ -163,7 +166,8 @@ int wafer_hip_gemm_mfma_residual(wafer_hip_context *ctx, const void *lhs,
  * gate rows 16j + [0,16) and rows 32j + 16 + [0,16) the up rows of the same
  * features; dst [m, features] = T(silu_mul(T(gate), T(up))), T = in_format
  * (BF16 or F16) -- the two narrowed products followed by the silu_mul region
- * (same bits); features a multiple of 16.  The region is the SwiGLU composition of
+ * (same bits, where wafer_hip_gemm_mfma does not split K for them: this entry
+ * never does); features a multiple of 16.  The region is the SwiGLU composition of
  * lib/Wafer/Conversion/TileToInstr/ComputeLowering.cpp:2555-2606 after two GEMMs. */
 int wafer_hip_gemm_mfma_swiglu(wafer_hip_context *ctx, const void *lhs,
                                const void *rhs_gu, void *dst, uint32_t m,
@@ -412,6 +416,11 @@ int wafer_hip_attention_prefill_masked(wafer_hip_context *ctx,
  * its own online state, then the states are folded left to right
  * (lib/Wafer/Transforms/Linalg/SpatialRegionMaterialization.cpp:2391-2430,
  * merge OnlineAttentionMaterialization.cpp:264-373) and finalised as FA.
+ * On small batches a chunk may be split over workgroups into states of its
+ * own, and runs of states (two of them from 5 states on, eight from 17) fold
+ * first, then the runs, left to right: the same merges in another
+ * association, so bits depend on the shape and the CU count, and repeat for a
+ * given shape.
  * q [batch, q_heads, 1, head_dim]; k/v caches [batch, kv_heads, kv_capacity,
  * head_dim] of which the first kv_len tokens are valid; o like q.
  * format BF16 or F16; head_dim 128; q_heads/kv_heads in {1, 2, 4, 8}.

@@ -20,7 +20,8 @@
 //    same work); wave w owns query tile w & 1 (32 queries) and key half
 //    w >> 1 (the even or the odd 64-key blocks); the two halves merge through
 //    LDS with the state merge of OnlineAttentionMaterialization.cpp:264-373.
-//    One wave per SIMD with the full 512-entry register file.
+//    One wave per SIMD with the full 512-entry register file (head_dim 64
+//    without a score region: two, see fa_waves).
 //    - S^T = K Q^T and O^T = V^T P^T on v_mfma_f32_32x32x16_{bf16,f16}: Q
 //      stays in VGPRs, K fragments are ds_read_b128 from LDS, V^T fragments
 //      come from row-major V through ds_read_b64_tr_b16, P^T feeds the B
@@ -240,9 +241,10 @@ __device__ inline int swz_v(int row) {
   return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1);
 }
 
-// Waves per SIMD: at head_dim 64 two workgroups fit a CU (256 registers per
-// wave, a few of them spilled outside the pipelined iteration), and one's
-// matrix work covers the other's softmax (4 x 8 heads x 1031: 34.5 -> 26.7 us);
+// Waves per SIMD: at head_dim 64 two workgroups fit a CU at 256 registers per
+// wave, and one's matrix work covers the other's softmax (4 x 8 heads x 1031:
+// 34.5 -> 26.7 us) although registers spill: 44 (MASK_CAUSAL, 180 bytes of
+// scratch a lane) and 182 (MASK_SELECT, 276 bytes);
 // the score region's mask operands do not fit that way (34.5 against 52.7 us at
 // 8 heads x 1024 with an additive mask).
 constexpr int fa_waves(int d, int mask) { return d == 64 && mask != MASK_GENERAL ? 2 : 1; }

@@ -9,7 +9,9 @@
 //   m = max(mL, mR), sL = ExpLp(mL - m), sR = ExpLp(mR - m),
 //   l = lL*sL + lR*sR, acc = accL*sL + accR*sR,
 // then finalised as FA: out = narrow(acc * (1/l)) to the BF16 or F16 storage.  GQA: q head h reads kv
-// head h / (q_heads / kv_heads).
+// head h / (q_heads / kv_heads).  On the chunk grid a chunk may be split into
+// several states, and runs of states fold before the runs do (fd_fold_d128):
+// the same merges in another association than the reference's left fold.
 //
 // The kernel is HBM-bound (every KV byte is read once, 4 B of traffic per
 // 4 FLOP), so the design goal is coalesced 128-bit streaming with enough
@@ -33,7 +35,8 @@
 //    heads over 8 KV heads, one sequence of 8192 keys: 20.4 -> 13.5 us; 8 over
 //    4, 3231 keys: 13.2 -> 9.2 us);
 //  * a decode step's new K / V row is read from the step's tensors and written
-//    to the cache by the wave that owns it, without a launch of its own.
+//    to the cache by the wave that owns it, without a launch of its own, where
+//    that is the faster way (appends_in_kernel).
 // Scores are tracked in the log2 domain (m2 = m * scale * log2e) so every
 // ExpLp becomes one exp2 of an fma; see fa_prefill.hip for the rounding note.
 #include "common.h"

@@ -23,7 +23,8 @@
 // rows divide by 4 and tile columns by 8), bounding the XCD's L2 working set.
 // For 16-bit operands, and int8 below 256x256 tiles, a 4-wave kernel (one wave
 // per SIMD, K slices moved by LDS DMA into a ring of 128 KiB) serves tiles
-// from 256x256 to 64x64, whichever the cost of their rounds says (pick_tile);
+// from 256x256 to 64x64, whichever the cost of their rounds says (pick_tile),
+// but for the products that the 8-wave kernel is faster at (gemm_route);
 // rows and columns that a tile does not divide end in a tile shifted back to
 // the edge.  Long-K grids of at most one round of 128x128 tiles may split K
 // over 4 workgroups of 256x256 tiles with a fold launch.  Products of few rows

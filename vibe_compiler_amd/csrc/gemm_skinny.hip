@@ -28,7 +28,10 @@
 // (14336->4096) at m 1.
 //
 // The order of the sum of one output depends on K alone (not on m, n, or the
-// epilogue), so the fused epilogues keep the bits of the unfused calls.
+// epilogue) for every product that this kernel serves, so the fused epilogues
+// keep the bits of the unfused calls.  It is not the k order of the tile kernels:
+// a row's bits differ between m 64 and 65 where n is large, and again where the
+// few-output rule ends.
 //
 // More rows on few columns take the same kernel on tiles of 64 x 32 (SwiGLU: 64 x
 // 64, the two products' columns), wherever those are one round of workgroups at
@@ -276,10 +279,10 @@ __global__ __launch_bounds__(64 * SKINNY_WAVES) void gemm_nt_skinny_kernel(GemmA
 }
 
 // ring depth that keeps a workgroup's LDS at 80 KiB (two per CU) where two
-// units at least fit, at most 8 units
+// units at least fit: 5 units at most (one tile of each)
 constexpr int ring_depth(int mt, int nt) {
   const int d = 80 / (SKINNY_WAVES * 2 * (mt + nt));
-  return d > 8 ? 8 : d < 2 ? 2 : d;
+  return d < 2 ? 2 : d;
 }
 
 template <int KIND, int OUT, int MT, int NT, int D = ring_depth(MT, NT)>
