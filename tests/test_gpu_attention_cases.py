@@ -589,3 +589,30 @@ def test_causal_middle_block(hip, oracle, Bn, Hq, Hkv, Sq, Skv, fmt):
     ot = torch.full((Bn, Sq, Hq, 128), 7.0, dtype=dt, device="cuda").permute(0, 2, 1, 3)
     hip.attention_prefill_strided(q, k, vt, ot, scale, causal=True, fmt=fmt)
     assert torch.equal(ot.contiguous().view(torch.int16), o.view(torch.int16))
+
+
+@pytest.mark.parametrize("fmt", [F16, BF16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("S", [1, 65, 1000])
+def test_head_dim_64_small_and_large_grids(hip, fmt, causal, S):
+    """head_dim 64 without masks: a grid of at most one workgroup per CU runs
+    one wave per SIMD, a larger one two.  Heads are independent, so the first
+    heads of a large call are a small call's, bit for bit, and both are float64
+    attention under the attention policy."""
+    say("head_dim 64 grids", fmt, causal, S)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    dt = torch.float16 if fmt == F16 else torch.bfloat16
+    cus, blocks = torch.cuda.get_device_properties(0).multi_processor_count, -(-S // 64)
+    small = cus // blocks
+    big = small + 1
+    q, k, v = (torch.randn(1, big, S, 64, generator=g, device="cuda").to(dt) for _ in range(3))
+    o, os = torch.full_like(q, 7.0), torch.full_like(q[:, :small], 7.0)
+    hip.attention_prefill_masked(q, k, v, o, 0.125, causal=causal, fmt=fmt)
+    hip.attention_prefill_masked(*(x[:, :small].contiguous() for x in (q, k, v)), os, 0.125, causal=causal, fmt=fmt)
+    assert torch.equal(o[:, :small].contiguous().view(torch.int16), os.view(torch.int16))
+    for h in (0, small - 1, big - 1):
+        x = q[0, h].double() @ k[0, h].double().t() * 0.125
+        if causal:
+            x.masked_fill_(torch.from_numpy(~band(S, S, 0)).cuda(), float("-inf"))
+        ref = torch.softmax(x, dim=-1) @ v[0, h].double()
+        attention_gate(o[0, h].float().cpu().numpy(), ref.float().cpu().numpy(), what=f"head {h}")

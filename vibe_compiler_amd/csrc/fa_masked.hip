@@ -249,9 +249,9 @@ __device__ inline int swz_v(int row) {
 // 8 heads x 1024 with an additive mask).
 constexpr int fa_waves(int d, int mask) { return d == 64 && mask != MASK_GENERAL ? 2 : 1; }
 
-template <typename T, int D, int MASK>
+template <typename T, int D, int MASK, int WAVES = fa_waves(D, MASK)>
 __global__ __launch_bounds__(THREADS)
-__attribute__((amdgpu_waves_per_eu(fa_waves(D, MASK), fa_waves(D, MASK)))) void fa_fwd(const FaArgs a) {
+__attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void fa_fwd(const FaArgs a) {
   constexpr int ROWB = 2 * D;            // bytes per K / V row
   constexpr int CH = ROWB / 16;          // 16-byte chunks per row
   constexpr int RPI = 64 / CH;           // rows per 1 KiB DMA instruction
@@ -1023,12 +1023,17 @@ int attention_prefill_masked(wafer_hip_context *ctx, uint32_t format, const void
     const bool two = fa_waves((int)head_dim, general ? MASK_GENERAL : select ? MASK_SELECT : MASK_CAUSAL) == 2;
     args.single = singles <= 0x7fffffffL && (two || cost_single < cost_pair);
     const dim3 grid((unsigned)(args.single ? singles : pairs));
+    // No second workgroup for a CU: head_dim 64 without masks takes all the
+    // registers, and no spills (us, two waves per SIMD / one: 4 x 28 heads of one
+    // query over 1000 keys 14.8 / 13.6, 32 heads x 512 10.8 / 10.0).
 #define FA_LAUNCH(TT, DD)                                                                              \
   do {                                                                                                 \
     if (general)                                                                                       \
       hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_GENERAL>), grid, dim3(THREADS), 0, ctx->stream, args);   \
     else if (select)                                                                                   \
       hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_SELECT>), grid, dim3(THREADS), 0, ctx->stream, args);    \
+    else if (DD == 64 && (long)grid.x <= cus)                                                          \
+      hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_CAUSAL, 1>), grid, dim3(THREADS), 0, ctx->stream, args); \
     else                                                                                               \
       hipLaunchKernelGGL((fa_fwd<TT, DD, MASK_CAUSAL>), grid, dim3(THREADS), 0, ctx->stream, args);    \
   } while (0)
