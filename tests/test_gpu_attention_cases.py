@@ -535,6 +535,11 @@ def test_far_scores_under_window_and_boolean_masks(hip, oracle, fmt, D, sign):
                 got = tof(oracle, fmt, run_masked(hip, fmt, qn, kn, vn, scale, **kw))[0, 0]
                 ref = hit.astype(np.float64) @ v[0, 0].double().numpy() / hit.sum(axis=1, keepdims=True)
                 assert hit.sum(axis=1).max() <= 2 and np.array_equal(got, ref), (a, b, scale, list(kw))
+    # as many heads as CUs: at head_dim 128 a workgroup takes both query blocks, one after the other
+    heads = torch.cuda.get_device_properties(0).multi_processor_count
+    one_head = run_masked(hip, fmt, qn, kn, vn, scale, keep=both)
+    all_heads = run_masked(hip, fmt, np.broadcast_to(qn, (1, heads, Sq, D)).copy(), kn, vn, scale, keep=both)
+    assert np.array_equal(all_heads, np.broadcast_to(one_head, all_heads.shape))
     # a far negative reference left for a near one: the last key's score is 0
     k[..., -1, :] = 0
     got = tof(oracle, fmt, run_masked(hip, fmt, qn, k.view(torch.int16).numpy().view(np.uint16), vn, scale,

@@ -144,8 +144,7 @@ __device__ inline float xor32_sum(float x) {
 // scale past 2.36e38 overflows.  Here the maximum is subtracted from t
 // itself, as the reference does.  Rare, so small rather than fast, and judged
 // after the merge: told apart inside the pipelined loop it cost calls without
-// such a row 10 to 25 %, judged there up to 6 % at head_dim 128 and up to 10 %
-// for masks per query at head_dim 64 (32 heads x 2048: 104 -> 113 us).
+// such a row 10 to 25 %, judged there 0 to 4 %.
 template <typename T, int D>
 __device__ inline void far_rows(const FaArgs &a, int bh, int qb, uint64_t rows) {
   const int quad = threadIdx.x & 3, row = (threadIdx.x >> 2) & 63, i = qb * QB + row;
@@ -244,7 +243,7 @@ __device__ inline int swz_v(int row) {
 // Waves per SIMD: at head_dim 64 two workgroups fit a CU at 256 registers per
 // wave, and one's matrix work covers the other's softmax (4 x 8 heads x 1031:
 // 34.5 -> 26.7 us) although registers spill: 44 (MASK_CAUSAL, 180 bytes of
-// scratch a lane) and 182 (MASK_SELECT, 276 bytes);
+// scratch a lane) and 131 (MASK_SELECT, 276 bytes);
 // the score region's mask operands do not fit that way (34.5 against 52.7 us at
 // 8 heads x 1024 with an additive mask).
 constexpr int fa_waves(int d, int mask) { return d == 64 && mask != MASK_GENERAL ? 2 : 1; }
@@ -616,6 +615,7 @@ __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void fa_fwd(const FaArgs a) {
       // weight, whose visible scores may have overflowed
       const bool far = (__builtin_fabsf(m_ref) > FAR_REF) & (m_ref != NOREF);
       sfar[wave][phase] = (uint32_t)__ballot(far | (acc[0][0] != acc[0][0]) | ((a.c > 1.0f) & (l == 0.0f)));
+      if (phase == 0) sfar[wave][1] = 0;
     }
     const f32x4 *px = (const f32x4 *)(xch + pw * (DT / 2) * 16 * 64 * 4);
     const int qi = q0 + l32;
@@ -820,14 +820,21 @@ __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void fa_fwd(const FaArgs a) {
   run_phase(0, qb_a, lo_a, ta, na_h, t);
   if (has_b) run_phase(1, qb_b, lo_b, tb, nb_h, t);
   if constexpr (MASK == MASK_SELECT) {  // (the merge's last barrier published sfar)
-    int id = blockIdx.x;
-    asm volatile("" : "+s"(id)::"memory");  // nothing of this is kept in registers over the loop above
-    const int pair2 = id / a.bh_count;
-    for (int phase = 0; phase < 2; ++phase) {
-      const int qb = phase ? pair2 : a.n_qblocks - 1 - pair2;
-      if (phase && (a.single || qb >= a.n_qblocks - 1 - pair2)) break;
-      const uint32_t r0 = sfar[0][phase] | sfar[2][phase], r1 = sfar[1][phase] | sfar[3][phase];
-      if (__builtin_expect(r0 | r1, 0)) far_rows<T, D>(a, id - pair2 * a.bh_count, qb, r0 | (uint64_t)r1 << 32);
+    uint32_t any = 0;
+    for (int x = 0; x < 8; ++x) any |= (&sfar[0][0])[x];
+    if (__builtin_expect(any != 0, 0)) {
+      // the arguments again, from memory: kept in registers over the loop above
+      // they cost masks per query at head_dim 64 8 % (32 heads x 2048: 104 -> 113 us)
+      auto *kp = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+      int id = blockIdx.x;
+      asm volatile("" : "+s"(kp), "+s"(id)::"memory");
+      FaArgs again;
+      __builtin_memcpy(&again, (const char *)kp, sizeof(FaArgs));
+      const int pair2 = id / again.bh_count, bh2 = id - pair2 * again.bh_count;
+      for (int phase = 0; phase < 2; ++phase) {
+        const uint32_t r0 = sfar[0][phase] | sfar[2][phase], r1 = sfar[1][phase] | sfar[3][phase];
+        if (r0 | r1) far_rows<T, D>(again, bh2, phase ? pair2 : again.n_qblocks - 1 - pair2, r0 | (uint64_t)r1 << 32);
+      }
     }
   }
 }
